@@ -1,0 +1,878 @@
+"""The measured cases: what a program built on this framework has it do.
+
+A program builds a network, lays it out once (its first step does that) and
+then streams samples through it in chunks: it runs the chunk's steps and looks
+at the network afterwards (the loss of every step, the unit columns, the
+weights and the optimizer's moments), to log, evaluate or checkpoint it. One
+pass is one such chunk on a network that has been laid out. Between passes the
+network goes on learning from where it stands.
+
+Kinds of case (``case["kind"]``):
+
+- ``stream``: a layered net with Zipf(1.1) source popularity, one sample per
+  step, MSE; ``rule`` the optimizer ("none": inference, the forward alone),
+  ``loop`` "step" (one call per step) or "scan" (``Driver.scan``, one chunk
+  per call), ``prune`` a PruneConn that kills about one edge in 2^20 per step;
+- ``pipeline``: a recurrent net whose units all fire every step (PIPELINE);
+- ``batch``: a sparse MLP on mini-batches;
+- ``dynamic``: a sparse MLP one sample per step whose smallest weights are
+  pruned and regrown by score once per chunk;
+- ``reservoir``: a recurrent net that proposes and claims new edges every
+  step, prunes silent units and spawns some every 100 steps;
+- ``head``: a sparse net with many outputs under softmax cross-entropy;
+- ``utility``: a net whose passes fold tuples under several monoids (weighted
+  input, largest contribution, in-degree), as continual-learning rules do.
+"""
+
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import torch
+
+import plastax_amd as px
+import plastax_amd.numpy as jnp
+
+GRAD = px.FieldSpec.float32("grad_pre_act")
+LOSSG = px.FieldSpec.float32("loss_grad")
+OUTDEG = px.FieldSpec.float32("out_degree")
+CONTRIB = px.FieldSpec.float32("contribution", 0.5)
+DEGREE = px.FieldSpec.float32("in_degree")
+LARGEST = px.FieldSpec.float32("largest")
+
+#: Optimizer state columns a pass returns beside the weights, by rule.
+STATE = {"none": (), "sgd": (), "momentum": ("opt/v",), "rmsprop": ("opt/v",), "adam": ("opt/m", "opt/v")}
+
+
+def listed():
+    return [
+        # One step of the small recurrent net as an online control loop calls
+        # it: a few launches over 16K edges, all latency.
+        {"name": "pipeline_step", "kind": "pipeline", "units": 1024, "edges": 16384, "inputs": 32, "outputs": 8,
+         "steps": 1, "loop": "step"},
+        # The same net learning from a recorded signal, 100 samples a call.
+        {"name": "pipeline_chunk", "kind": "pipeline", "units": 1024, "edges": 16384, "inputs": 32, "outputs": 8,
+         "steps": 100, "loop": "scan"},
+        # The layered net at 1/64 of its full width (1M edges), in chunks.
+        {"name": "zipf_small", "kind": "stream", "layers": 8, "width": 2048, "fan": 73, "rule": "adam", "steps": 32,
+         "loop": "scan", "prune": False},
+        # An odd width, a shallower net, another rule, one call per step.
+        {"name": "zipf_odd", "kind": "stream", "layers": 5, "width": 30011, "fan": 37, "rule": "rmsprop", "steps": 32,
+         "loop": "step", "prune": False},
+        # The full net: 8 x 131,072 units, 2^26 edges.
+        {"name": "zipf_full", "kind": "stream", "layers": 8, "width": 131072, "fan": 73, "rule": "adam", "steps": 48,
+         "loop": "step", "prune": False},
+        # A quarter of it with edges pruned every step (tombstones in the rows).
+        {"name": "zipf_prune", "kind": "stream", "layers": 8, "width": 32768, "fan": 73, "rule": "adam", "steps": 32,
+         "loop": "step", "prune": True},
+        # The sparse MLP (2.0M edges) on mini-batches of 256.
+        {"name": "mlp_batch", "kind": "batch", "sizes": "784,4096,4096,10", "keep": 0.1, "batch": 256, "rule": "adam",
+         "steps": 8},
+        # Odd layer sizes, a batch that is no multiple of 4, another rule.
+        {"name": "mlp_batch_odd", "kind": "batch", "sizes": "301,1003,777,37", "keep": 0.2, "batch": 70,
+         "rule": "momentum", "steps": 8},
+        # The sparse MLP one sample per step, pruned and regrown every 100.
+        {"name": "mlp_dynamic", "kind": "dynamic", "sizes": "784,4096,4096,10", "keep": 0.1, "shortlist": 32,
+         "steps": 100},
+        # The growing reservoir: 4M edges in 16M slots, growth every step.
+        {"name": "reservoir", "kind": "reservoir", "units": 65536, "edges": 1 << 22, "inputs": 256, "capacity": 262144,
+         "steps": 20},
+        # Many labels: 65,536 outputs under softmax cross-entropy.
+        {"name": "head_softmax", "kind": "head", "inputs": 2048, "hidden": 1024, "outputs": 65536, "fan": 16,
+         "steps": 16},
+        # Tuple accumulators in both directions of a mid-sized sparse MLP.
+        {"name": "utility", "kind": "utility", "sizes": "784,2048,2048,10", "keep": 0.1, "steps": 16},
+    ]
+
+
+def _log(rng, lo, hi):
+    """A whole number, uniform over the logarithm of [lo, hi]."""
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["stream", "stream", "stream", "pipeline", "batch", "batch", "dynamic", "reservoir", "head",
+                       "utility"])
+    if kind == "stream":
+        prune = rng.random() < 0.2
+        fan = _log(rng, 4, 80)
+        return {"kind": kind, "layers": rng.randint(3, 8), "width": _log(rng, 8 * fan, 100000), "fan": fan,
+                "rule": "adam" if prune else rng.choice(["adam", "adam", "sgd", "momentum", "rmsprop", "none"]),
+                "steps": rng.randint(8, 48), "loop": "step" if prune else rng.choice(["step", "scan"]), "prune": prune}
+    if kind == "pipeline":
+        units = _log(rng, 200, 20000)
+        steps = rng.choice([1, rng.randint(2, 100)])
+        return {"kind": kind, "units": units, "edges": units * rng.randint(4, 32), "inputs": rng.randint(1, 64),
+                "outputs": rng.randint(1, 64), "steps": steps, "loop": "step" if steps == 1 else "scan"}
+    if kind == "batch":
+        sizes = [_log(rng, 50, 1000), _log(rng, 200, 4096), _log(rng, 200, 4096), _log(rng, 2, 100)]
+        return {"kind": kind, "sizes": ",".join(map(str, sizes)), "keep": round(rng.uniform(0.05, 0.25), 3),
+                "batch": _log(rng, 8, 256), "rule": rng.choice(["adam", "sgd", "momentum", "rmsprop", "none"]),
+                "steps": rng.randint(1, 8)}
+    if kind == "dynamic":
+        sizes = [_log(rng, 100, 800), _log(rng, 300, 4096), _log(rng, 300, 4096), _log(rng, 4, 50)]
+        return {"kind": kind, "sizes": ",".join(map(str, sizes)), "keep": round(rng.uniform(0.05, 0.1), 3),
+                "shortlist": rng.randint(8, 32), "steps": rng.randint(20, 100)}
+    if kind == "reservoir":
+        units = _log(rng, 2000, 65536)
+        return {"kind": kind, "units": units, "edges": units * rng.randint(16, 64), "inputs": rng.randint(8, 256),
+                "capacity": 4 * units, "steps": rng.randint(4, 20)}
+    if kind == "head":
+        return {"kind": kind, "inputs": _log(rng, 200, 4000), "hidden": _log(rng, 200, 4000),
+                "outputs": _log(rng, 1000, 131072), "fan": rng.randint(4, 32), "steps": rng.randint(4, 16)}
+    sizes = [_log(rng, 100, 800), _log(rng, 200, 2048), _log(rng, 200, 2048), _log(rng, 4, 50)]
+    return {"kind": kind, "sizes": ",".join(map(str, sizes)), "keep": round(rng.uniform(0.05, 0.15), 3),
+            "steps": rng.randint(4, 16)}
+
+
+# --------------------------------------------------------------------------
+# Policies
+# --------------------------------------------------------------------------
+class _Tanh(px.ForwardPass):
+    combine = px.monoid.sum_
+
+    def map(self, u, dst, src, c, cid, g):
+        return c[px.WEIGHT, cid] * u[px.ACTIVATION, src]
+
+    def apply(self, u, i, g, acc):
+        return px.UnitWrite.of((px.ACTIVATION, jnp.tanh(acc)))
+
+
+class _Relu(_Tanh):
+    def apply(self, u, i, g, acc):
+        return px.UnitWrite.of((px.ACTIVATION, jnp.maximum(acc, jnp.float32(0.0))))
+
+
+class _TanhBack(px.BackwardPass):
+    combine = px.monoid.sum_
+
+    def map(self, u, src, dst, c, cid, g):
+        return c[px.WEIGHT, cid] * u[GRAD, dst]
+
+    def apply(self, u, i, g, acc):
+        a = u[px.ACTIVATION, i]
+        return px.UnitWrite.of((GRAD, (acc + u[LOSSG, i]) * (jnp.float32(1.0) - a * a)))
+
+
+class _ReluBack(_TanhBack):
+    def apply(self, u, i, g, acc):
+        gate = jnp.where(u[px.ACTIVATION, i] > 0, jnp.float32(1.0), jnp.float32(0.0))
+        return px.UnitWrite.of((GRAD, (acc + u[LOSSG, i]) * gate))
+
+
+class _Mse(px.Loss):
+    seed_field = LOSSG
+
+    def calculate_loss(self, u, outputs, targets, g):
+        d = u.gather(px.ACTIVATION, outputs) - targets
+        return jnp.sum(jnp.float32(0.5) * d * d), d
+
+
+class _HashPrune(px.PruneConn):
+    """About one edge in 2^20 per step, from its ids and the step."""
+
+    def predicate(self, u, c, cid, g):
+        h = c[px.FROM_ID, cid] * jnp.int32(7) + c[px.TO_ID, cid] * jnp.int32(13) + g["step"]
+        return (h % jnp.int32(1048573)) == jnp.int32(0)
+
+
+class _SmallPrune(px.PruneConn):
+    def predicate(self, u, c, cid, g):
+        return jnp.abs(c[px.WEIGHT, cid]) < g["tau"]
+
+
+class _UtilityForward(px.ForwardPass):
+    combine = (px.monoid.sum_, px.monoid.max_, px.monoid.sum_)
+
+    def map(self, u, dst, src, c, cid, g):
+        return (c[px.WEIGHT, cid] * u[px.ACTIVATION, src], jnp.abs(c[px.WEIGHT, cid]) * c[CONTRIB, cid],
+                jnp.float32(1.0))
+
+    def apply(self, u, i, g, acc):
+        s, m, n = acc
+        return px.UnitWrite.of((px.ACTIVATION, jnp.tanh(s) + m * jnp.float32(0.01)), (DEGREE, n), (LARGEST, m))
+
+
+class _UtilityBack(px.BackwardPass):
+    combine = px.monoid.sum_
+
+    def map(self, u, src, dst, c, cid, g):
+        a = u[px.ACTIVATION, src]
+        return c[px.WEIGHT, cid] * u[GRAD, dst] * (jnp.float32(1.0) + a * a)
+
+    def apply(self, u, i, g, acc):
+        a = u[px.ACTIVATION, i]
+        return px.UnitWrite.of((GRAD, (acc + u[LOSSG, i]) * (jnp.float32(1.0) - a * a)))
+
+
+class _CountOut(px.BackwardPass):
+    combine = px.monoid.sum_
+
+    def map(self, u, src, dst, c, cid, g):
+        return jnp.float32(1.0)
+
+    def apply(self, u, i, g, acc):
+        return px.UnitWrite.of((OUTDEG, acc))
+
+
+class _PruneSilent(px.PruneUnit):
+    def predicate(self, u, i, g):
+        return u[OUTDEG, i] == jnp.float32(0.0)
+
+
+def _optimizer(rule):
+    return {"sgd": lambda: px.optim.sgd(1e-3, GRAD), "momentum": lambda: px.optim.momentum(1e-4, 0.9, GRAD),
+            "adam": lambda: px.optim.adam(1e-3, GRAD), "rmsprop": lambda: px.optim.rmsprop(1e-3, GRAD)}[rule]()
+
+
+def _network(fwd, back=None, loss_=None, rule="none", units=(), conns=(), **more):
+    """A network class of these policies (an inference net has no backward)."""
+    if rule == "none":
+        body = {"forward_pass": fwd, "extra_unit_fields": tuple(units), "extra_conn_fields": tuple(conns)}
+    else:
+        opt = _optimizer(rule)
+        body = {"forward_pass": fwd, "backward_pass": back, "loss": loss_, "update_conn": opt.update_conn(),
+                "extra_unit_fields": (GRAD, LOSSG, *units), "extra_conn_fields": (*conns, *opt.state_fields)}
+    body.update(more)
+    return type("Net", (px.Network,), body)
+
+
+# --------------------------------------------------------------------------
+# Inputs (all from the seed alone)
+# --------------------------------------------------------------------------
+DEV = "cuda"
+
+
+def _gen(seed, salt):
+    return torch.Generator(device=DEV).manual_seed(1000003 * int(seed) + salt)
+
+
+def _zipf_layer(gen, n_src, n_dst, fan):
+    """(source, destination) of one layer pair: about ``fan`` distinct sources
+    per destination (one more for every 7th), drawn by Zipf(1.1) popularity
+    over a random order of the sources."""
+    cdf = torch.cumsum(torch.arange(1, n_src + 1, dtype=torch.float64, device=DEV) ** -1.1, 0)
+    cdf /= cdf[-1].clone()
+    perm = torch.randperm(n_src, generator=gen, device=DEV)
+    m = 2 * fan + 16
+    src, dst = [], []
+    for r0 in range(0, n_dst, 32768):
+        rows = torch.arange(r0, min(r0 + 32768, n_dst), device=DEV)
+        u = torch.rand((rows.numel(), m), generator=gen, device=DEV, dtype=torch.float64)
+        d = torch.searchsorted(cdf, u, right=True).clamp_(max=n_src - 1)
+        srt, order = torch.sort(d, dim=1, stable=True)
+        fresh = torch.ones_like(srt, dtype=torch.bool)
+        fresh[:, 1:] = srt[:, 1:] != srt[:, :-1]
+        first = torch.empty_like(fresh).scatter_(1, order, fresh)
+        need = fan + (rows % 7 == 0).long()
+        take = first & (torch.cumsum(first, 1) <= need[:, None])
+        src.append(perm[d[take]])
+        dst.append(rows[:, None].expand(-1, m)[take])
+    return torch.cat(src), torch.cat(dst)
+
+
+def _stream_edges(case, seed):
+    """Per bucket (source, destination, weight) in slot order."""
+    n_l, w = case["layers"], case["width"]
+    gen = _gen(seed, 1)
+    out = []
+    for layer in range(n_l - 1):
+        src, dst = _zipf_layer(gen, w, w, case["fan"])
+        out.append(_in_slots(gen, src + layer * w, dst + (layer + 1) * w, n_l * w, case["fan"]))
+    return out
+
+
+def _head_edges(case, seed):
+    """Input -> hidden -> outputs, about ``fan`` sources each."""
+    gen = _gen(seed, 2)
+    sizes = [case["inputs"], case["hidden"], case["outputs"]]
+    base = [0, sizes[0], sizes[0] + sizes[1], sum(sizes)]
+    out = []
+    for layer in range(2):
+        src, dst = _zipf_layer(gen, sizes[layer], sizes[layer + 1], case["fan"])
+        out.append(_in_slots(gen, src + base[layer], dst + base[layer + 1], base[-1], case["fan"]))
+    return out
+
+
+def _in_slots(gen, src, dst, n, fan):
+    """Source-major slot order and weights N(0, 1/fan)."""
+    key, _ = torch.sort(src * n + dst)
+    w = torch.randn(key.numel(), generator=gen, device=DEV) / math.sqrt(fan)
+    return torch.div(key, n, rounding_mode="floor").int(), (key % n).int(), w
+
+
+def _sizes(case):
+    return [int(s) for s in case["sizes"].split(",")]
+
+
+def _mlp_edges(case, seed):
+    """The sparse MLP's edges on the host: a random share ``keep`` of each
+    pair of consecutive layers' edges, at least one into every unit."""
+    sizes = _sizes(case)
+    rng = np.random.default_rng([int(seed), 3])
+    base = np.concatenate([[0], np.cumsum(sizes)])
+    src, dst = [], []
+    for k in range(len(sizes) - 1):
+        m = rng.random((sizes[k], sizes[k + 1]), dtype=np.float32)
+        j = np.arange(sizes[k + 1])
+        m[j % sizes[k], j] = -1.0
+        take = max(round(case["keep"] * m.size), j.size)
+        a, b = np.divmod(np.argpartition(m.ravel(), take - 1)[:take], j.size)
+        src.append(base[k] + a)
+        dst.append(base[k + 1] + b)
+    src, dst = np.concatenate(src).astype(np.int32), np.concatenate(dst).astype(np.int32)
+    fan = np.bincount(dst, minlength=int(base[-1]))
+    w = (rng.standard_normal(src.size) / np.sqrt(fan[dst])).astype(np.float32)
+    return base, src, dst, w
+
+
+def _recurrent_edges(case, seed):
+    """Uniform random edges without self-loops, in slot order."""
+    gen = _gen(seed, 4)
+    n, m = case["units"], case["edges"]
+    src = torch.randint(0, n, (m,), generator=gen, device=DEV)
+    dst = torch.randint(0, n - 1, (m,), generator=gen, device=DEV)
+    dst = dst + (dst >= src)
+    return _in_slots(gen, src, dst, n, m / n)
+
+
+def _samples(case, seed, steps, n_in, n_out, labels=False):
+    """Inputs N(0, 1) and targets: one-hot labels, or values of the inputs."""
+    gen = _gen(seed, 5)
+    shape = (steps, case["batch"]) if "batch" in case else (steps,)
+    x = torch.randn((*shape, n_in), generator=gen, device=DEV)
+    if labels:
+        at = torch.randint(0, n_out, shape, generator=gen, device=DEV)
+        return x, torch.nn.functional.one_hot(at, n_out).float()
+    pick = torch.randint(0, n_in, (n_out,), generator=gen, device=DEV)
+    sign = torch.randint(0, 2, (n_out,), generator=gen, device=DEV).float() * 2 - 1
+    return x, torch.tanh(x[..., pick] * sign)
+
+
+# --------------------------------------------------------------------------
+# Networks on the GPU
+# --------------------------------------------------------------------------
+_DTYPES = {"float32": torch.float32, "int32": torch.int32, "bool": torch.uint8}
+
+
+def _columns(specs, n, given):
+    """One column per spec: the given values, then the spec's default."""
+    out = {}
+    for s in specs:
+        col = torch.full((n,), float(s.default) if str(s.dtype) == "float32" else int(s.default),
+                         dtype=_DTYPES[str(s.dtype)], device=DEV)
+        if s.name in given:
+            col[: given[s.name].numel()] = given[s.name].to(col.dtype)
+        out[s.name] = col
+    return out
+
+
+def _on_gpu(net, n, edges, levels, caps, input_ids, output_ids, globals_):
+    """The state of ``net`` over ``edges`` (one (source, destination, weight)
+    per bucket, in slot order), laid out as ``NetworkBuilder.from_edges`` lays
+    it out; built on the GPU, since tens of millions of edges are sorted here."""
+    slots = n if net.unit_capacity is None else net.unit_capacity
+    ufields = (px.ACTIVATION, px.LEVEL, *((px.PRUNED,) if net.unit_capacity is not None else ()),
+               *net.extra_unit_fields)
+    cfields = (px.FROM_ID, px.TO_ID, px.DEAD, px.WEIGHT, *net.extra_conn_fields)
+    units = _columns(ufields, slots, {"level": levels, "pruned": torch.zeros(n, device=DEV)})
+    conns = tuple(_columns(cfields, cap, {"from_id": s, "to_id": d, "weight": w,
+                                          "dead": torch.zeros(s.numel(), device=DEV)})
+                  for (s, d, w), cap in zip(edges, caps))
+    pipeline = net.propagation is px.Propagation.PIPELINE
+    static = px.NetworkStatic(num_units=slots, propagation=net.propagation, unit_fields=ufields, conn_fields=cfields,
+                              level_capacities=tuple(caps), kahn_max_depth=net.kahn_max_depth,
+                              input_ids=tuple(input_ids), output_ids=tuple(output_ids),
+                              capacity_align=None if pipeline else 256,
+                              capacity_headroom=3.0 if pipeline else 0.0, seed=net.seed)
+    state = px.NetworkState(units, conns, globals_, tail_start=edges[0][0].numel() if pipeline else 0)
+    return static, state
+
+
+def _layer_caps(case):
+    """Slots per bucket: room for every destination's sources (a few find
+    fewer distinct ones than they ask for), a multiple of 256."""
+    into = [case["width"]] * (case["layers"] - 1) if case["kind"] == "stream" else [case["hidden"], case["outputs"]]
+    return [-(-max(n * case["fan"] + -(-n // 7), 64) // 256) * 256 for n in into]
+
+
+def _layer_levels(sizes):
+    return torch.repeat_interleave(torch.arange(len(sizes), device=DEV), torch.tensor(sizes, device=DEV))
+
+
+# --------------------------------------------------------------------------
+# prepare / run
+# --------------------------------------------------------------------------
+def prepare(case, seed):
+    """The network, laid out by its first step (scan: its first chunk), and
+    the chunk of samples a pass streams through it."""
+    s = _PREPARE[case["kind"]](case, seed)
+    s.update(case=dict(case), count=0)
+    if case.get("loop") == "scan" and case.get("rule") != "none":
+        s["driver"] = px.Driver(s.pop("net"), s.pop("static"), s.pop("state"))
+        s["driver"].scan(px.StepInputs(s["x"], s["t"]))
+    else:
+        s["step"] = px.make_step(s.pop("net"), s.pop("static"), batch_size=case.get("batch"))
+        _steps(s, 1)
+    return s
+
+
+def _prepare_stream(case, seed):
+    n_l, w = case["layers"], case["width"]
+    more = {"prune_conn": _HashPrune()} if case["prune"] else {}
+    net = _network(_Tanh(), _TanhBack(), _Mse(), case["rule"], **more)
+    edges = _stream_edges(case, seed)
+    static, state = _on_gpu(net, n_l * w, edges, _layer_levels([w] * n_l), _layer_caps(case), range(w),
+                            range((n_l - 1) * w, n_l * w), {"step": np.int32(0)} if case["prune"] else None)
+    x, t = _samples(case, seed, case["steps"], w, w)
+    return {"net": net, "static": static, "state": state, "x": x, "t": t}
+
+
+def _prepare_head(case, seed):
+    sizes = [case["inputs"], case["hidden"], case["outputs"]]
+    net = _network(_Tanh(), _TanhBack(), px.SoftmaxCrossEntropyLoss(LOSSG), "adam")
+    edges = _head_edges(case, seed)
+    static, state = _on_gpu(net, sum(sizes), edges, _layer_levels(sizes), _layer_caps(case), range(sizes[0]),
+                            range(sizes[0] + sizes[1], sum(sizes)), None)
+    x, t = _samples(case, seed, case["steps"], sizes[0], sizes[2], labels=True)
+    return {"net": net, "static": static, "state": state, "x": x, "t": t}
+
+
+def _prepare_pipeline(case, seed):
+    net = _network(_Tanh(), _TanhBack(), _Mse(), "sgd", propagation=px.Propagation.PIPELINE)
+    src, dst, w = (v.cpu().numpy() for v in _recurrent_edges(case, seed))
+    n = case["units"]
+    static, state = px.NetworkBuilder.from_edges(net, n, src, dst, weights=w, input_ids=range(case["inputs"]),
+                                                 output_ids=range(n - case["outputs"], n), globals_=None)
+    x, t = _samples(case, seed, case["steps"], case["inputs"], case["outputs"])
+    return {"net": net, "static": static, "state": state, "x": x, "t": t}
+
+
+def _prepare_mlp(case, seed):
+    base, src, dst, w = _mlp_edges(case, seed)
+    more, headroom, g = {}, 0.0, None
+    if case["kind"] == "batch":
+        net = _network(_Relu(), _ReluBack(), px.SoftmaxCrossEntropyLoss(LOSSG), case["rule"],
+                       batch_reduction=px.MeanFloatFirstRest())
+    elif case["kind"] == "utility":
+        net = _network(_UtilityForward(), _UtilityBack(), px.SoftmaxCrossEntropyLoss(LOSSG), "adam",
+                       units=(DEGREE, LARGEST), conns=(CONTRIB,))
+    else:
+        net = _network(_Tanh(), _TanhBack(), px.SoftmaxCrossEntropyLoss(LOSSG), "adam", prune_conn=_SmallPrune(),
+                       add_conn=_regrowth(case["shortlist"], case["steps"]))
+        headroom, g = 0.1, {"tau": np.float32(0.0)}
+        more = {"kill": 2 * case["shortlist"] ** 2}
+    static, state = px.NetworkBuilder.from_edges(net, int(base[-1]), src, dst, weights=w, input_ids=range(base[1]),
+                                                 output_ids=range(base[-2], base[-1]), globals_=g,
+                                                 capacity_headroom=headroom)
+    x, t = _samples(case, seed, case["steps"], int(base[1]), int(base[-1] - base[-2]), labels=True)
+    return {"net": net, "static": static, "state": state, "x": x, "t": t, **more}
+
+
+def _regrowth(side, every):
+    """Up to ``side`` x ``side`` new edges per level, by |act[src] * grad[dst]|
+    over a shortlist, every ``every`` steps."""
+
+    class Grow(px.ScoreAddConn):
+        candidates = "shortlist_per_level"
+        shortlist_size = side
+        direction = "deeper"
+        max_level_gap = 1
+        dedupe_live = True
+        max_new_per_level = side * side
+        trigger = ("every", every)
+
+        def score(self, u, src, dst, g):
+            return jnp.abs(u[px.ACTIVATION, src] * u[GRAD, dst])
+
+        def importance(self, u, i, g):
+            return jnp.abs(u[GRAD, i]) + jnp.abs(u[px.ACTIVATION, i])
+
+        def init(self, u, src, dst, g):
+            return px.ConnWrite.of((px.WEIGHT, jnp.float32(0.0)))
+
+    return Grow()
+
+
+def _prepare_reservoir(case, seed):
+    n = case["units"]
+    lo, hi = n // 64, n // 64 + 16
+
+    class Spawn(px.AddUnit):
+        def spawn(self, u, parent, g):
+            return (parent >= lo) & (parent < hi) & (g["spawn"] > jnp.float32(0.0)), jnp.int32(0)
+
+        def init(self, u, child, parent, g):
+            return px.UnitWrite.of((px.ACTIVATION, u[px.ACTIVATION, parent] * jnp.float32(0.5)))
+
+    class Propose(px.ProposeAddConn):
+        proposer = "per_unit"
+        proposals_per_proposer = 4
+        max_new_per_level = 16
+        max_level_gap = 1 << 20
+
+        def propose(self, u, i, j, g, rng):
+            return jnp.asarray(i, jnp.int32), rng.uniform_int(n).astype(jnp.int32), rng.uniform()
+
+        def init(self, u, src, dst, g):
+            return px.ConnWrite.of((px.WEIGHT, jnp.float32(0.01)))
+
+    net = _network(_Tanh(), units=(OUTDEG,), backward_pass=_CountOut(), prune_unit=_PruneSilent(), add_unit=Spawn(),
+                   add_conn=Propose(), propagation=px.Propagation.PIPELINE, unit_capacity=case["capacity"])
+    edges = [_recurrent_edges(case, seed)]
+    cap = 1 << (4 * case["edges"] - 1).bit_length()
+    # Every unit but the inputs lies on or behind a cycle: the builder's levels
+    # are 1 for the units that an input feeds and 0 for the others.
+    src, dst, _ = edges[0]
+    levels = torch.zeros(n, device=DEV)
+    levels[dst[src < case["inputs"]].long()] = 1
+    levels[: case["inputs"]] = 0
+    static, state = _on_gpu(net, n, edges, levels, [cap], range(case["inputs"]), range(n - 16, n),
+                            {"spawn": np.float32(0.0)})
+    x, _ = _samples(case, seed, case["steps"], case["inputs"], 16)
+    return {"net": net, "static": static, "state": state, "x": x, "t": None}
+
+
+_PREPARE = {"stream": _prepare_stream, "head": _prepare_head, "pipeline": _prepare_pipeline, "batch": _prepare_mlp,
+            "utility": _prepare_mlp, "dynamic": _prepare_mlp, "reservoir": _prepare_reservoir}
+
+
+def _globals(s, state):
+    """What the program sets before a step: the step's number for the hashed
+    prune, the spawn flag every 100 steps, the pruning threshold (of the
+    ``kill`` smallest weights) once per chunk."""
+    case, k = s["case"], s["count"]
+    if case.get("prune"):
+        state.globals_ = {"step": np.int32(k)}
+    elif case["kind"] == "reservoir":
+        state.globals_ = {"spawn": np.float32(k % 100 == 0)}
+    elif case["kind"] == "dynamic":
+        if k % case["steps"] == 0:
+            w = torch.cat([b["weight"][b["dead"] == 0].abs() for b in state.conns])
+            state.globals_ = {"tau": np.float32(torch.kthvalue(w, min(s["kill"], w.numel() // 4)).values.item())}
+        elif k % case["steps"] == 1:
+            state.globals_ = {"tau": np.float32(0.0)}
+
+
+def _steps(s, count):
+    """``count`` steps, one call each; the losses."""
+    state, losses = s["state"], []
+    for i in range(count):
+        _globals(s, state)
+        t = s["t"]
+        r = s["step"](state, px.StepInputs(s["x"][i], None if t is None else t[i]))
+        state = r.state
+        losses.append(r.loss)
+        s["count"] += 1
+    s["state"] = state
+    return losses
+
+
+def run(s):
+    """One chunk, then the network as the program looks at it."""
+    case = s["case"]
+    out = {}
+    if "driver" in s:
+        out["loss"] = s["driver"].scan(px.StepInputs(s["x"], s["t"]))
+        state = s["driver"].state
+    else:
+        losses = _steps(s, case["steps"])
+        if _rule(case) != "none":
+            out["loss"] = torch.stack(losses)
+        state = s["state"]
+    units = state.units
+    out["units"] = {n: units[n] for n in _unit_names(case)}
+    conns = _conn_names(case)
+    if conns:
+        out["conns"] = [{n: b[n] for n in conns} for b in state.conns]
+    return out
+
+
+def _rule(case):
+    return {"pipeline": "sgd", "dynamic": "adam", "head": "adam", "utility": "adam",
+            "reservoir": "none"}.get(case["kind"], case.get("rule"))
+
+
+def _unit_names(case):
+    if case["kind"] == "reservoir":
+        return ("activation", "out_degree", "pruned")
+    if _rule(case) == "none":
+        return ("activation",)
+    more = ("in_degree", "largest") if case["kind"] == "utility" else ()
+    return ("activation", "grad_pre_act", "loss_grad", *more)
+
+
+def _conn_names(case):
+    if case["kind"] == "reservoir":
+        return ("from_id", "to_id", "dead", "weight")
+    if _rule(case) == "none":
+        return ()
+    more = ("from_id", "to_id") if case["kind"] == "dynamic" else ()
+    return (*more, *(("dead",) if case.get("prune") or case["kind"] == "dynamic" else ()), "weight",
+            *STATE[_rule(case)])
+
+
+# --------------------------------------------------------------------------
+# work / tolerance
+# --------------------------------------------------------------------------
+def _edge_count(case):
+    """(edges, edges whose backward terms are folded, units)."""
+    kind = case["kind"]
+    if kind == "stream":
+        per = case["width"] * (case["fan"] + 1 / 7)
+        return per * (case["layers"] - 1), per * (case["layers"] - 2), case["width"] * case["layers"]
+    if kind == "head":
+        return (case["hidden"] + case["outputs"]) * (case["fan"] + 1 / 7), case["outputs"] * (case["fan"] + 1 / 7), \
+            case["inputs"] + case["hidden"] + case["outputs"]
+    if kind in ("pipeline", "reservoir"):
+        return case["edges"], case["edges"], case["units"]
+    sizes = _sizes(case)
+    per = [case["keep"] * a * b for a, b in zip(sizes, sizes[1:])]
+    return sum(per), sum(per[1:]), sum(sizes)
+
+
+def work(case):
+    """A step reads each edge's two ids, weight and optimizer state once and
+    writes the weight and the state once (inference: reads ids and weight);
+    it reads and writes the unit columns once. Products and sums: two per edge
+    and sample in each direction, two for the batch-mean gradient, the rule's
+    (3 to 16) per edge."""
+    edges, folded, units = _edge_count(case)
+    rule, batch = _rule(case), case.get("batch", 1)
+    state = len(STATE[rule])
+    train = rule != "none"
+    per_edge = 8 + 4 * (1 + state) * (2 if train else 1)
+    per_unit = (4 + (12 if train else 4)) * (1 if batch == 1 else batch)
+    if case["kind"] == "reservoir":  # the growth's proposals and the outdegree count
+        per_unit += 16
+    flops = 2 * batch * (edges + (folded if train else 0))
+    if train:
+        flops += edges * (2 * batch + {"sgd": 2, "momentum": 4, "rmsprop": 8, "adam": 16}[rule])
+    return {"bytes": case["steps"] * (edges * per_edge + units * per_unit), "flops": case["steps"] * flops}
+
+
+def tolerance(case):
+    """Sums in 32 bits, in another order: up to 3e-6 off 64 bits over the
+    listed and drawn cases. Adam and RMSProp divide by the root of the squared
+    gradient: where a gradient nearly cancels, the step's sign is a matter of
+    rounding and a single entry differs by up to a step's length. ReLU units
+    (batch) whose input nearly cancels pass or stop a whole gradient: 8e-4 off
+    64 bits where one of them turns over."""
+    if case["kind"] == "batch":
+        return {"rel": 3e-3, "max": 0.5}
+    return {"rel": 1e-5, "max": 0.05 if _rule(case) in ("adam", "rmsprop") else 1e-3}
+
+
+# --------------------------------------------------------------------------
+# exact: the same passes in 64 bits, in plain torch
+# --------------------------------------------------------------------------
+def _apply_rule(rule, e, g, t, live):
+    """One step of the rule on an edge list ``e`` (constants as the rules keep
+    them, in 32 bits)."""
+    f = lambda v: float(np.float32(v))  # noqa: E731
+    keep = {k: e[k] for k in ("weight", "opt/m", "opt/v") if k in e}
+    if rule == "sgd":
+        e["weight"] = e["weight"] - f(1e-3) * g
+    elif rule == "momentum":
+        e["opt/v"] = f(0.9) * e["opt/v"] + g
+        e["weight"] = e["weight"] - f(1e-4) * e["opt/v"]
+    elif rule == "adam":
+        e["opt/m"] = f(0.9) * e["opt/m"] + f(1 - 0.9) * g
+        e["opt/v"] = f(0.999) * e["opt/v"] + f(1 - 0.999) * g * g
+        m, v = e["opt/m"] / (1 - f(0.9) ** t), e["opt/v"] / (1 - f(0.999) ** t)
+        e["weight"] = e["weight"] - f(1e-3) * (m / (torch.sqrt(v) + f(1e-8)))
+    elif rule == "rmsprop":
+        e["opt/v"] = f(0.9) * e["opt/v"] + f(1 - 0.9) * g * g
+        e["weight"] = e["weight"] - f(1e-3) * g / torch.sqrt(e["opt/v"] + f(1e-8))
+    if live is not None:
+        for k, old in keep.items():
+            e[k] = torch.where(live, e[k], old)
+
+
+def _edge_dicts(edges, rule):
+    out = []
+    for s, d, w in edges:
+        e = {"src": s.long(), "dst": d.long(), "weight": w.double()}
+        e.update({n: torch.zeros_like(e["weight"]) for n in STATE[rule]})
+        e["by_dst"] = torch.sort(e["dst"], stable=True)
+        out.append(e)
+    return out
+
+
+def _run_sums(ids, v, units):
+    """Sums of v over the runs of equal ids (ascending), for the unit ids in
+    the slice ``units``: differences of the running sum (no atomics)."""
+    at = torch.searchsorted(ids, torch.arange(units.start, units.stop + 1, device=DEV))
+    run = torch.nn.functional.pad(torch.cumsum(v, 0), (1, 0))
+    return run[at[1:]] - run[at[:-1]]
+
+
+def _to_dst(e, v, units):
+    """v summed by destination, for the units of a slice."""
+    ids, order = e["by_dst"]
+    return _run_sums(ids, v[order], units)
+
+
+def _to_src(e, v, units):
+    """v summed by source (the edges' own order)."""
+    return _run_sums(e["src"], v, units)
+
+
+def _exact_layered(case, seed, sizes, edges, labels, caps):
+    """Layered nets one sample per step: stream, head, utility."""
+    rule, utility = _rule(case), case["kind"] == "utility"
+    n, k = sum(sizes), case["steps"]
+    es = _edge_dicts(edges, rule)
+    base = np.concatenate([[0], np.cumsum(sizes)])
+    layer = [slice(int(a), int(b)) for a, b in zip(base, base[1:])]
+    x, t = _samples(case, seed, k, sizes[0], sizes[-1], labels=labels)
+    x, t = x.double(), t.double()
+    zero = lambda: torch.zeros(n, dtype=torch.float64, device=DEV)  # noqa: E731
+    act, grad, lossg, deg, big = zero(), zero(), zero(), zero(), zero()
+    live = [torch.ones_like(e["src"], dtype=torch.bool) if case.get("prune") else None for e in es]
+    scan = case.get("loop") == "scan" and rule != "none"
+    todo = list(range(k)) * 2 if scan else [0, *range(k)]
+    losses = []
+    for number, i in enumerate(todo):
+        act[layer[0]] = x[i]
+        for b, e in enumerate(es):
+            term = e["weight"] * act[e["src"]]
+            if live[b] is not None:
+                term = torch.where(live[b], term, 0.0)
+            s = _to_dst(e, term, layer[b + 1])
+            a = torch.tanh(s)
+            if utility:
+                m = torch.full((n,), -math.inf, dtype=torch.float64, device=DEV)
+                m = m.scatter_reduce(0, e["dst"], e["weight"].abs() * 0.5, "amax")[layer[b + 1]]
+                deg[layer[b + 1]] = _to_dst(e, torch.ones_like(term), layer[b + 1])
+                big[layer[b + 1]] = m
+                a = a + m * float(np.float32(0.01))
+            act[layer[b + 1]] = a
+        if rule == "none":
+            continue
+        out = act[layer[-1]]
+        if labels:
+            lossg[layer[-1]] = torch.softmax(out, 0) - t[i]
+            losses.append(-(torch.log_softmax(out, 0) * t[i]).sum())
+        else:
+            lossg[layer[-1]] = out - t[i]
+            losses.append(0.5 * ((out - t[i]) ** 2).sum())
+        grad[layer[-1]] = lossg[layer[-1]] * (1 - out * out)
+        for b in range(len(es) - 1, -1, -1):
+            e = es[b]
+            if b > 0:
+                term = e["weight"] * grad[e["dst"]]
+                if live[b] is not None:
+                    term = torch.where(live[b], term, 0.0)
+                if utility:
+                    term = term * (1 + act[e["src"]] ** 2)
+                a = act[layer[b]]
+                grad[layer[b]] = (_to_src(e, term, layer[b]) + lossg[layer[b]]) * (1 - a * a)
+            _apply_rule(rule, e, grad[e["dst"]] * act[e["src"]], number + 1, live[b])
+            if live[b] is not None:
+                live[b] &= (e["src"] * 7 + e["dst"] * 13 + number) % 1048573 != 0
+    return _answer(case, losses[-k:], {"activation": act, "grad_pre_act": grad, "loss_grad": lossg, "in_degree": deg,
+                                       "largest": big}, es, caps)
+
+
+def _answer(case, losses, units, es, caps):
+    out = {"units": {n: units[n] for n in _unit_names(case)}}
+    if _rule(case) != "none":
+        out["loss"] = torch.stack(losses)
+        names = _conn_names(case)
+        out["conns"] = []
+        for b, e in enumerate(es):
+            pad = (0, caps[b] - e["src"].numel())
+            out["conns"].append({n: torch.nn.functional.pad(e[n], pad) if n in e else None for n in names})
+    return out
+
+
+def _split(base, src, dst, w):
+    """The MLP's edges per layer, in slot order."""
+    out = []
+    for k in range(len(base) - 2):
+        m = (src >= base[k]) & (src < base[k + 1])
+        o = np.lexsort((dst[m], src[m]))
+        out.append(tuple(torch.from_numpy(np.ascontiguousarray(v[m][o])).to(DEV) for v in (src, dst, w)))
+    return out
+
+
+def _policy_caps(edges):
+    return [max(64, 1 << (int(s.numel()) - 1).bit_length()) for s, _, _ in edges]
+
+
+def _exact_batch(case, seed):
+    rule, sizes, k, B = _rule(case), _sizes(case), case["steps"], case["batch"]
+    base, src, dst, w = _mlp_edges(case, seed)
+    edges = _split(base, src, dst, w)
+    es = _edge_dicts(edges, rule)
+    x, t = _samples(case, seed, k, sizes[0], sizes[-1], labels=True)
+    x, t = x.double(), t.double()
+    names = ("activation", "grad_pre_act", "loss_grad")
+    units = {n: torch.zeros(int(base[-1]), dtype=torch.float64, device=DEV) for n in names}
+    losses = []
+    for number, i in enumerate([0, *range(k)]):
+        acts, dense = [x[i].t()], []
+        for b, e in enumerate(es):
+            m = torch.zeros((sizes[b + 1], sizes[b]), dtype=torch.float64, device=DEV)
+            m[e["dst"] - int(base[b + 1]), e["src"] - int(base[b])] = e["weight"]
+            dense.append(m)
+            acts.append(torch.relu(m @ acts[-1]))
+        units["activation"] = torch.cat([a.mean(1) for a in acts])
+        if rule == "none":
+            continue
+        out = acts[-1]
+        lg = torch.softmax(out, 0) - t[i].t()
+        losses.append(-(torch.log_softmax(out, 0) * t[i].t()).sum(0).mean())
+        grads = [None] * len(acts)
+        grads[-1] = lg * (out > 0)
+        for b in range(len(es) - 1, 0, -1):
+            grads[b] = (dense[b].t() @ grads[b + 1]) * (acts[b] > 0)
+        for b, e in enumerate(es):
+            mean = grads[b + 1] @ acts[b].t() / B
+            _apply_rule(rule, e, mean[e["dst"] - int(base[b + 1]), e["src"] - int(base[b])], number + 1, None)
+        grads[0] = torch.zeros_like(acts[0])
+        units["grad_pre_act"] = torch.cat([v.mean(1) for v in grads])
+        units["loss_grad"][int(base[-2]):] = lg.mean(1)
+    return _answer(case, losses[-k:], units, es, _policy_caps(edges))
+
+
+def _exact_pipeline(case, seed):
+    n, k = case["units"], case["steps"]
+    edges = [_recurrent_edges(case, seed)]
+    (e,) = es = _edge_dicts(edges, "sgd")
+    x, t = _samples(case, seed, k, case["inputs"], case["outputs"])
+    x, t = x.double(), t.double()
+    act, grad, lossg = (torch.zeros(n, dtype=torch.float64, device=DEV) for _ in range(3))
+    losses, every = [], slice(0, n)
+    for i in (list(range(k)) * 2 if case["loop"] == "scan" else [0, *range(k)]):
+        act[: case["inputs"]] = x[i]
+        new = torch.tanh(_to_dst(e, e["weight"] * act[e["src"]], every))
+        new[: case["inputs"]] = x[i]
+        act = new
+        d = act[n - case["outputs"]:] - t[i]
+        lossg[n - case["outputs"]:] = d
+        losses.append(0.5 * (d * d).sum())
+        grad = (_to_src(e, e["weight"] * grad[e["dst"]], every) + lossg) * (1 - act * act)
+        _apply_rule("sgd", e, grad[e["dst"]] * act[e["src"]], 0, None)
+    return _answer(case, losses[-k:], {"activation": act, "grad_pre_act": grad, "loss_grad": lossg}, es,
+                   _policy_caps(edges))
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind == "stream":
+        return _exact_layered(case, seed, [case["width"]] * case["layers"], _stream_edges(case, seed), False,
+                              _layer_caps(case))
+    if kind == "head":
+        sizes = [case["inputs"], case["hidden"], case["outputs"]]
+        return _exact_layered(case, seed, sizes, _head_edges(case, seed), True, _layer_caps(case))
+    if kind == "pipeline":
+        return _exact_pipeline(case, seed)
+    if kind == "batch":
+        return _exact_batch(case, seed)
+    if kind == "utility":
+        edges = _split(*_mlp_edges(case, seed))
+        return _exact_layered(case, seed, _sizes(case), edges, True, _policy_caps(edges))
+    return None  # what is pruned and grown follows 32-bit comparisons
