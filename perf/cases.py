@@ -550,7 +550,8 @@ def _globals(s, state):
     elif case["kind"] == "dynamic":
         if k % case["steps"] == 0:
             w = torch.cat([b["weight"][b["dead"] == 0].abs() for b in state.conns])
-            state.globals_ = {"tau": np.float32(torch.kthvalue(w, min(s["kill"], w.numel() // 4)).values.item())}
+            small = torch.topk(w, min(s["kill"], w.numel() // 4), largest=False).values
+            state.globals_ = {"tau": np.float32(small.max().item())}
         elif k % case["steps"] == 1:
             state.globals_ = {"tau": np.float32(0.0)}
 
