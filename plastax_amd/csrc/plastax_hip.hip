@@ -52,8 +52,8 @@ using plx_detail::fail;
 namespace {
 
 template <int M, bool PRUNE>
-__global__ __launch_bounds__(kFwdBlock) void k_forward(plx_forward_desc d) {
-  forward_body<M, PRUNE, SiteInterp>(d);
+__global__ __launch_bounds__(kFwdBlock) void k_forward(plx_forward_desc d, int rows) {
+  forward_body<M, PRUNE, SiteInterp>(d, rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -1523,7 +1523,7 @@ int dispatch_rule(const plx_tile_desc& d, size_t lds, hipStream_t s) {
 }  // namespace
 
 int plx_detail::forward_launch_shape(const plx_forward_desc* d, const char* who, unsigned* grid,
-                                     unsigned* block) {
+                                     unsigned* block, int* rows) {
   const std::string w(who);
   *grid = 0;
   *block = kFwdBlock;
@@ -1539,8 +1539,9 @@ int plx_detail::forward_launch_shape(const plx_forward_desc* d, const char* who,
     return fail(PLX_ERR_INVALID, (w + ": fin.level and fin.is_input are required").c_str());
   if (d->prune_prog && (!d->prune_sink || d->num_units <= 0))
     return fail(PLX_ERR_INVALID, (w + ": prune_prog needs prune_sink and num_units").c_str());
-  const unsigned nblk = grid_for(d->nrows, kFwdRows);
   const unsigned cap = static_cast<unsigned>(cu_count() * kFwdPerCU);
+  *rows = fwd_block_rows(d->nrows, cu_count());
+  const unsigned nblk = grid_for(d->nrows, *rows);
   *grid = nblk < cap ? nblk : cap;
   return PLX_OK;
 }
@@ -1569,34 +1570,35 @@ int plx_struct_sizes(int64_t* out, int32_t n) {
 
 int plx_forward_bucket(const plx_forward_desc* d, void* stream) {
   unsigned grid = 0, block = 0;
-  const int rc = plx_detail::forward_launch_shape(d, "plx_forward_bucket", &grid, &block);
+  int rows = 0;
+  const int rc = plx_detail::forward_launch_shape(d, "plx_forward_bucket", &grid, &block, &rows);
   if (rc || grid == 0) return rc;
   const bool prune = d->prune_prog != nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (d->monoid) {
     case PLX_MONOID_SUM:
       if (prune)
-        k_forward<PLX_MONOID_SUM, true><<<grid, kFwdBlock, 0, s>>>(*d);
+        k_forward<PLX_MONOID_SUM, true><<<grid, kFwdBlock, 0, s>>>(*d, rows);
       else
-        k_forward<PLX_MONOID_SUM, false><<<grid, kFwdBlock, 0, s>>>(*d);
+        k_forward<PLX_MONOID_SUM, false><<<grid, kFwdBlock, 0, s>>>(*d, rows);
       break;
     case PLX_MONOID_PROD:
       if (prune)
-        k_forward<PLX_MONOID_PROD, true><<<grid, kFwdBlock, 0, s>>>(*d);
+        k_forward<PLX_MONOID_PROD, true><<<grid, kFwdBlock, 0, s>>>(*d, rows);
       else
-        k_forward<PLX_MONOID_PROD, false><<<grid, kFwdBlock, 0, s>>>(*d);
+        k_forward<PLX_MONOID_PROD, false><<<grid, kFwdBlock, 0, s>>>(*d, rows);
       break;
     case PLX_MONOID_MAX:
       if (prune)
-        k_forward<PLX_MONOID_MAX, true><<<grid, kFwdBlock, 0, s>>>(*d);
+        k_forward<PLX_MONOID_MAX, true><<<grid, kFwdBlock, 0, s>>>(*d, rows);
       else
-        k_forward<PLX_MONOID_MAX, false><<<grid, kFwdBlock, 0, s>>>(*d);
+        k_forward<PLX_MONOID_MAX, false><<<grid, kFwdBlock, 0, s>>>(*d, rows);
       break;
     case PLX_MONOID_MIN:
       if (prune)
-        k_forward<PLX_MONOID_MIN, true><<<grid, kFwdBlock, 0, s>>>(*d);
+        k_forward<PLX_MONOID_MIN, true><<<grid, kFwdBlock, 0, s>>>(*d, rows);
       else
-        k_forward<PLX_MONOID_MIN, false><<<grid, kFwdBlock, 0, s>>>(*d);
+        k_forward<PLX_MONOID_MIN, false><<<grid, kFwdBlock, 0, s>>>(*d, rows);
       break;
     default: return fail(PLX_ERR_UNSUPPORTED, "plx_forward_bucket: unknown monoid");
   }

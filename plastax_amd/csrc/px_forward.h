@@ -329,8 +329,8 @@ __device__ __forceinline__ int32_t ld_uniform(const int32_t* p, int64_t i) {
 }
 
 // ---------------------------------------------------------------------------
-// Forward: rows (destination units) are cut into blocks of kFwdRows, one row
-// per lane of the first kFwdRows lanes. Each workgroup of a persistent grid
+// Forward: rows (destination units) are cut into blocks of at most kFwdRows
+// (fwd_block_rows), one row per lane of a block's first lanes. Each workgroup of a persistent grid
 // (kFwdPerCU per CU) takes a contiguous run of blocks, whose positions are
 // contiguous too, and streams them through LDS in windows of kFwdWin terms
 // with 16-byte loads of FROM_ID and WEIGHT (map = weight * x[src], table hits
@@ -365,6 +365,27 @@ constexpr int kFwdQuads = PLX_FWD_QUADS;  // 16-byte quads per thread per window
 constexpr int kFwdWin = 4 * kFwdQuads * kFwdBlock;
 constexpr int kFwdPerCU = PLX_FWD_PER_CU;  // workgroups per CU in the persistent grid
 
+// Rows per block of a launch over nrows rows on ncu CUs. A level of up to
+// kFwdRows * kFwdPerCU * ncu rows (131,072 on 256 CUs) is cut so that every
+// workgroup slot gets one block: with 256-row blocks a level of 4,096 rows
+// kept 16 CUs busy (410 edges a row: 105K edges one after another), and what
+// is left after the cut is one block's chain of memory latencies. Below eight
+// rows a block the rule stops at one workgroup per CU: such blocks hold too
+// few edges for a second one to hide anything. Per launch, 256-row blocks
+// before, this rule after: 4,096 rows of 410 edges 83 -> 10.5 us; 2,048 rows
+// of 73 17.1 -> 7.0; 30,011 of 37 14.0 -> 9.6; 32,768 of 73 20.6 -> 13.2;
+// 131,072 of 73 (still 256 rows) 26.7 -> 26.2 by the fold's longer reads.
+// Twice as many blocks (two waves of workgroups) were slower everywhere
+// (10.9 / 13.3 / 15.0 us for the last three but one), and so were tables cut
+// to a share of the block's edges (7.5 against 7.2).
+inline int fwd_block_rows(int nrows, int ncu) {
+  const int two = (nrows + kFwdPerCU * ncu - 1) / (kFwdPerCU * ncu);
+  const int one = (nrows + ncu - 1) / ncu;
+  const int few = one < 8 ? one : 8;
+  const int rows = two > few ? two : few;
+  return rows < kFwdRows ? rows : kFwdRows;
+}
+
 // A window's raw columns: FROM_ID and WEIGHT quads, DEAD bytes.
 struct FwdRaw {
   int4 sv[kFwdQuads];
@@ -398,20 +419,21 @@ __device__ __forceinline__ uint8_t prune_at(const plx_forward_desc& d, int64_t p
   return out[0] != 0u;
 }
 
-// The body of a forward launch (kFwdBlock lanes per workgroup). PRUNE: the
+// The body of a forward launch (kFwdBlock lanes per workgroup; `rows` rows
+// per block, at most kFwdRows). PRUNE: the
 // PruneConn predicate of every visited position goes to prune_sink (see
 // plx_forward_desc), evaluated by Prog.
 template <int M, bool PRUNE, class Prog>
-__device__ __forceinline__ void forward_body(const plx_forward_desc& d) {
+__device__ __forceinline__ void forward_body(const plx_forward_desc& d, int rows) {
   __shared__ __align__(16) float buf[2][kFwdWin];
   __shared__ float tbl[kFwdTbl > 0 ? kFwdTbl : 1];
-  const int nblk = (d.nrows + kFwdRows - 1) / kFwdRows;
+  const int nblk = (d.nrows + rows - 1) / rows;
   const int b0 = static_cast<int>(static_cast<int64_t>(blockIdx.x) * nblk / gridDim.x);
   const int b1 = static_cast<int>(static_cast<int64_t>(blockIdx.x + 1) * nblk / gridDim.x);
   if (b0 >= b1) return;  // uniform over the workgroup
   const int tlen = kFwdTbl > 0 ? min(d.tbl_len, kFwdTbl) : 0;
   const float ident = Mono<M>::id();
-  auto row_end = [&](int blk) { return d.row_ptr[min((blk + 1) * kFwdRows, d.nrows)]; };
+  auto row_end = [&](int blk) { return d.row_ptr[min((blk + 1) * rows, d.nrows)]; };
 
   // Windows in order: every block has at least one (an empty block's
   // window holds nothing). ee_next is the end of the block after the last
@@ -529,15 +551,17 @@ __device__ __forceinline__ void forward_body(const plx_forward_desc& d) {
   bool has = false;
   RowPre pre;
   auto setup_rows = [&]() {
-    r = fb * kFwdRows + static_cast<int>(threadIdx.x);
-    has = threadIdx.x < kFwdRows && r < d.nrows;
+    r = fb * rows + static_cast<int>(threadIdx.x);
+    has = static_cast<int>(threadIdx.x) < rows && r < d.nrows;
     my_b = has ? d.row_ptr[r] : 0;
     my_e = has ? d.row_ptr[r + 1] : 0;
     if (has) pre = prefetch_row(d.row_unit, r, d.fin, d.apply);
   };
   float s = ident;
   // The lane's row over window w held in `in`: the unaligned head one term
-  // at a time, then aligned 16-byte runs, the last one padded with the
+  // at a time, then aligned 16-byte runs (eight reads in flight per step
+  // while the row is long: with few rows a block the fold is the window's
+  // serial part), the last one padded with the
   // identity past the row's end (for every monoid that leaves the running
   // value's bits unchanged: a sum that starts at +0 never holds -0).
   auto fold = [&](const float* in, const FwdWin& w) {
@@ -548,6 +572,18 @@ __device__ __forceinline__ void forward_body(const plx_forward_desc& d) {
     int j = lo;
     const int a = min((lo + 3) & ~3, hi);
     for (; j < a; ++j) s = Mono<M>::op(s, in[j]);
+    for (; j + 32 <= hi; j += 32) {
+      float4 x[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[k] = *reinterpret_cast<const float4*>(in + j + 4 * k);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        s = Mono<M>::op(s, x[k].x);
+        s = Mono<M>::op(s, x[k].y);
+        s = Mono<M>::op(s, x[k].z);
+        s = Mono<M>::op(s, x[k].w);
+      }
+    }
     for (; j + 8 <= hi; j += 8) {
       const float4 x0 = *reinterpret_cast<const float4*>(in + j);
       const float4 x1 = *reinterpret_cast<const float4*>(in + j + 4);
@@ -571,7 +607,7 @@ __device__ __forceinline__ void forward_body(const plx_forward_desc& d) {
 
   // Prologue: window 0's loads, the table, the first rows, window 0's
   // terms (window 1's loads go out meanwhile).
-  FwdWin wc{b0, 0, d.row_ptr[b0 * kFwdRows], row_end(b0)};
+  FwdWin wc{b0, 0, d.row_ptr[b0 * rows], row_end(b0)};
   wc.w0 = wc.eb & ~3;
   FwdRaw A, B;
   load(A, wc);

@@ -1245,8 +1245,8 @@ std::string site_source(const plx_site_desc& d) {
 // (px_forward.h's forward_body), for monoid m.
 std::string forward_prune_source(const plx_site_desc& d, int32_t m) {
   return site_gen_source(d, "px_forward.h") +
-         "extern \"C\" __global__ __launch_bounds__(kFwdBlock) void plx_fwd_prune_kernel(plx_forward_desc d) {\n"
-         "  forward_body<" + std::to_string(m) + ", true, SiteGen>(d);\n}\n";
+         "extern \"C\" __global__ __launch_bounds__(kFwdBlock) void plx_fwd_prune_kernel(plx_forward_desc d, int rows) {\n"
+         "  forward_body<" + std::to_string(m) + ", true, SiteGen>(d, rows);\n}\n";
 }
 
 int site_rtc_compile(const std::string& src, const char* csrc_dir, const std::string& arch, std::vector<char>* code) {
@@ -1414,12 +1414,13 @@ int plx_forward_bucket_compiled(void* handle, const plx_forward_desc* d, void* s
     return fail(PLX_ERR_INVALID,
                 "plx_forward_bucket_compiled: ids_logical / ids_physical are not set as in the compiled shape");
   unsigned grid = 0, block = 0;
-  const int rc = plx_detail::forward_launch_shape(d, "plx_forward_bucket_compiled", &grid, &block);
+  int rows = 0;
+  const int rc = plx_detail::forward_launch_shape(d, "plx_forward_bucket_compiled", &grid, &block, &rows);
   if (rc || grid == 0) return rc;
   int dev = -1;
   if (hipGetDevice(&dev) != hipSuccess || dev != cs->dev)
     return fail(PLX_ERR_INVALID, "plx_forward_bucket_compiled: the kernel was compiled for another device");
-  void* args[] = {const_cast<plx_forward_desc*>(d)};
+  void* args[] = {const_cast<plx_forward_desc*>(d), &rows};
   if (hipModuleLaunchKernel(cs->fn, grid, 1, 1, block, 1, 1, 0, static_cast<hipStream_t>(stream), args, nullptr) !=
       hipSuccess)
     return fail(PLX_ERR_HIP, "plx_forward_bucket_compiled: launch failed");
