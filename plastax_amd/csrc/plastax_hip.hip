@@ -45,6 +45,7 @@ int check_launch(const char* what) {
 }  // namespace plx_detail
 
 using plx_detail::check_launch;
+using plx_detail::cu_count;
 using plx_detail::fail;
 
 #include "px_forward.h"
@@ -1444,20 +1445,6 @@ inline unsigned grid_for(int64_t n, int block) {
   return static_cast<unsigned>((n + block - 1) / block);
 }
 
-// The current device's CU count (queried once per device; 256 on MI355X).
-int cu_count() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] <= 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 // A program's sizes are in range; fields read at a fixed unit only where
 // the kernel honours them (the loss) and only among the program's fields.
 bool program_ok(const plx_program& p, bool fixed_ok = false) {
@@ -1521,6 +1508,19 @@ int dispatch_rule(const plx_tile_desc& d, size_t lds, hipStream_t s) {
 }
 
 }  // namespace
+
+int plx_detail::cu_count() {
+  static int cached[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cached[dev] <= 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      n = 256;
+    cached[dev] = n;
+  }
+  return cached[dev];
+}
 
 int plx_detail::forward_launch_shape(const plx_forward_desc* d, const char* who, unsigned* grid,
                                      unsigned* block, int* rows) {

@@ -18,6 +18,9 @@ int check_launch(const char* what);
 // rows, nothing to launch) of *block lanes, *rows rows per block.
 int forward_launch_shape(const plx_forward_desc* d, const char* who, unsigned* grid, unsigned* block,
                          int* rows);
+
+// The current device's CU count (queried once per device; 256 on MI355X).
+int cu_count();
 }  // namespace plx_detail
 #endif
 
