@@ -402,16 +402,12 @@ PLX_EXPORT int plx_update_batch_tiles(const plx_update_desc* d, const plx_batch_
                                       void* stream);
 
 /* Batched losses: sample b's outputs at ids[k] * B + b, targets[b * n_out +
- * k], loss into losses[b]; the per-sample fold is plx_loss_elementwise's /
- * plx_loss_softmax_ce's. partials: B * ceil(n_out / 256) floats. */
+ * k], loss into losses[b]; the per-sample fold is plx_loss_elementwise's.
+ * partials: B * ceil(n_out / 256) floats. */
 PLX_EXPORT int plx_loss_elementwise_batch(int32_t n_out, const int32_t* output_ids,
                                           const float* targets, const plx_program* term,
                                           float* seed_field, float* partials, float* losses,
                                           int32_t batch, void* stream);
-PLX_EXPORT int plx_loss_softmax_ce_batch(int32_t n_out, const int32_t* output_ids,
-                                         const float* act, const float* targets,
-                                         float* seed_field, float* losses, int32_t batch,
-                                         void* stream);
 
 /* StepResult.loss of a batched step (step.py:466): (0 + l_0 + ... + l_{B-1}) / B. */
 PLX_EXPORT int plx_batch_mean(int32_t batch, const float* losses, float* out, void* stream);
@@ -447,10 +443,15 @@ PLX_EXPORT int plx_loss_elementwise(int32_t n_out, const int32_t* output_ids,
 
 /* SoftmaxCrossEntropyLoss (traits.py:204-250): max, sum of exp(a - max) in
  * 256-output pieces, seed = exp(z)/s - t, loss = piecewise fold of
- * t*(log s - z). Runs in one workgroup. */
+ * t*(log s - z), at most 262144 outputs. Sample b of batch (1: a streaming
+ * step): outputs at ids[k] * batch + b, targets[b * n_out + k], loss into
+ * losses[b]. Up to PLX_SOFTMAX_ONE outputs run in one workgroup per sample;
+ * more need partials: 3 * batch * ceil(n_out / 256) floats of scratch. */
+#define PLX_SOFTMAX_ONE 4096
 PLX_EXPORT int plx_loss_softmax_ce(int32_t n_out, const int32_t* output_ids,
                         const float* act, const float* targets,
-                        float* seed_field, float* loss_out, void* stream);
+                        float* seed_field, float* partials, float* losses,
+                        int32_t batch, void* stream);
 
 /* Fill n floats with a value (identity accumulators). */
 PLX_EXPORT int plx_fill_f32(int64_t n, float value, float* dst, void* stream);

@@ -18,13 +18,14 @@ LIB_PATH = pathlib.Path(
     or pathlib.Path(__file__).resolve().parent / "libplastax_hip.so"
 )
 
-ABI_VERSION = 28  # plx_abi_version() of the library these mirrors describe
+ABI_VERSION = 29  # plx_abi_version() of the library these mirrors describe
 
 PLX_MAX_INSTR = 48
 PLX_MAX_CONST = 32
 PLX_MAX_FIELDS = 8
 PLX_MAX_OUTS = 4
 PLX_MAX_TBL = 8192
+PLX_SOFTMAX_ONE = 4096
 PLX_MAX_SINSTR = 160
 PLX_MAX_SCONST = 32
 PLX_MAX_SFIELDS = 8
@@ -493,7 +494,7 @@ _SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
         c_i32,
         [c_i32, c_vp, c_vp, ctypes.POINTER(plx_program), c_vp, c_vp, c_vp, c_vp],
     ),
-    "plx_loss_softmax_ce": (c_i32, [c_i32, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]),
+    "plx_loss_softmax_ce": (c_i32, [c_i32, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i32, c_vp]),
     "plx_fill_f32": (c_i32, [c_i64, c_f32, c_vp, c_vp]),
     "plx_forward_batch": (c_i32, [ctypes.POINTER(plx_forward_desc), c_i32, c_vp]),
     "plx_backward_batch": (c_i32, [ctypes.POINTER(plx_bwd_batch_desc), c_vp]),
@@ -505,7 +506,6 @@ _SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
         c_i32,
         [c_i32, c_vp, c_vp, ctypes.POINTER(plx_program), c_vp, c_vp, c_vp, c_i32, c_vp],
     ),
-    "plx_loss_softmax_ce_batch": (c_i32, [c_i32, c_vp, c_vp, c_vp, c_vp, c_vp, c_i32, c_vp]),
     "plx_batch_mean": (c_i32, [c_i32, c_vp, c_vp, c_vp]),
     "plx_reduce_batch": (c_i32, [c_i64, c_i32, c_i32, c_i32, c_vp, c_vp, c_vp]),
     "plx_philox32": (c_i32, [c_i64, c_vp, c_vp, c_vp, c_vp]),

@@ -39,7 +39,7 @@ from plastax_amd._layout import Arena
 from plastax_amd._plan import Plan, program_struct
 from plastax_amd._types import ACTIVATION
 from plastax_amd.state import NetworkState, NetworkStatic
-from plastax_amd.step import StepFn, StepInputs, StepResult, _stream
+from plastax_amd.step import StepFn, StepInputs, StepResult, _stream, softmax_partials
 from plastax_amd.traits import Reduction, batch_written_reduction
 
 _REDUCE = {Reduction.MEAN: 0, Reduction.SUM: 1, Reduction.FIRST: 2}
@@ -288,10 +288,12 @@ class BatchedStepFn(StepFn):
             lp = plan.loss
             ids = consts["output_ids"].data_ptr()
             if lp.kind == "softmax":
+                parts = softmax_partials(n_out, B, dev)
                 _lib.check(
-                    lib.plx_loss_softmax_ce_batch(n_out, ids, ub[ACTIVATION.name].data_ptr(), t.data_ptr(),
-                                                  ub[lp.seed_field].data_ptr(), losses.data_ptr(), B, stream),
-                    "plx_loss_softmax_ce_batch",
+                    lib.plx_loss_softmax_ce(n_out, ids, ub[ACTIVATION.name].data_ptr(), t.data_ptr(),
+                                            ub[lp.seed_field].data_ptr(), None if parts is None else parts.data_ptr(),
+                                            losses.data_ptr(), B, stream),
+                    "plx_loss_softmax_ce",
                 )
             else:
                 parts = torch.empty(B * (n_out // 256 + 1) + 1, dtype=torch.float32, device=dev)

@@ -1305,6 +1305,27 @@ __global__ void k_fill(int64_t n, float value, float* dst) {
 }
 
 constexpr int kPiece = 256;
+constexpr int kPieceStride = kPiece + 4;  // a piece's LDS row: 16-byte aligned, the pieces' rows four banks apart
+
+// s + v[0] + ... + v[len - 1] in order (v in LDS, 16-byte aligned): the chain
+// of adds is serial, so its reads go out 32 values ahead of it.
+__device__ __forceinline__ float fold_in_order(const float* v, int len, float s) {
+  int j = 0;
+  for (; j + 32 <= len; j += 32) {
+    float4 x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = *reinterpret_cast<const float4*>(v + j + 4 * k);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      s = s + x[k].x;
+      s = s + x[k].y;
+      s = s + x[k].z;
+      s = s + x[k].w;
+    }
+  }
+  for (; j < len; ++j) s = s + v[j];
+  return s;
+}
 
 // One 256-output piece per workgroup: each thread runs the loss program for
 // one output (out slot 0, the seed, lands at the output's unit id; slot 1 is
@@ -1314,7 +1335,7 @@ constexpr int kPiece = 256;
 __global__ __launch_bounds__(kPiece) void k_loss_pieces(int32_t n_out, const int32_t* ids,
                                                        const float* targets, plx_program P,
                                                        float* piece_sums, int32_t B) {
-  __shared__ float terms[kPiece];
+  __shared__ __align__(16) float terms[kPiece];
   const int b = blockIdx.y;
   const int k = blockIdx.x * kPiece + threadIdx.x;
   if (k < n_out) {
@@ -1323,18 +1344,15 @@ __global__ __launch_bounds__(kPiece) void k_loss_pieces(int32_t n_out, const int
         run_program(P, u, load_loss_fields(P, u, b), 0.0f, targets[static_cast<int64_t>(b) * n_out + k], true);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const int len = min(kPiece, n_out - static_cast<int>(blockIdx.x) * kPiece);
-    float s = 0.0f;
-    for (int j = 0; j < len; ++j) s = s + terms[j];
-    piece_sums[static_cast<int64_t>(b) * gridDim.x + blockIdx.x] = s;
-  }
+  if (threadIdx.x == 0)
+    piece_sums[static_cast<int64_t>(b) * gridDim.x + blockIdx.x] =
+        fold_in_order(terms, min(kPiece, n_out - static_cast<int>(blockIdx.x) * kPiece), 0.0f);
 }
 
 // Folds n piece sums in order from +0.0 into *out, staging them through LDS
 // (workgroup b: sums[b * n ..] into out[b]).
 __global__ __launch_bounds__(1024) void k_fold_sums(int32_t n, const float* sums, float* out) {
-  __shared__ float buf[1024];
+  __shared__ __align__(16) float buf[1024];
   sums += static_cast<int64_t>(blockIdx.x) * n;
   out += blockIdx.x;
   float s = 0.0f;
@@ -1342,79 +1360,168 @@ __global__ __launch_bounds__(1024) void k_fold_sums(int32_t n, const float* sums
     const int len = min(1024, n - base);
     if (static_cast<int>(threadIdx.x) < len) buf[threadIdx.x] = sums[base + threadIdx.x];
     __syncthreads();
-    if (threadIdx.x == 0)
-      for (int j = 0; j < len; ++j) s = s + buf[j];
+    if (threadIdx.x == 0) s = fold_in_order(buf, len, s);
     __syncthreads();
   }
   if (threadIdx.x == 0) *out = 0.0f + s;
 }
 
+// Softmax cross-entropy. The exponentials, seeds and loss terms are computed
+// side by side; what stays serial is each 256-output piece's sum and the sum
+// over the pieces, both in order.
+//
+// Up to kSoftmaxOne outputs one workgroup does a sample alone (k_softmax_ce);
+// its time is a few launches' latency, so one launch is best. Beyond that a
+// workgroup per piece and three launches (k_softmax_max, _sum, _seed) and the
+// fold of the pieces' losses: 65,536 outputs 335 us in one workgroup that
+// summed its pieces from global memory, one lane each.
 constexpr int kSoftmaxMaxPieces = 1024;
+constexpr int kSoftmaxOne = PLX_SOFTMAX_ONE;  // outputs of the one-workgroup form
+constexpr int kSoftmaxPer = kSoftmaxOne / 1024;  // outputs per thread there
+static_assert(kSoftmaxOne % kPiece == 0 && kSoftmaxPer * 1024 == kSoftmaxOne, "whole pieces, whole threads");
 
-// Workgroup b is sample b: unit u at u * B + b, targets[b * n ..], loss_out[b].
-__global__ __launch_bounds__(1024) void k_softmax_ce(int32_t n, const int32_t* ids,
-                                                     const float* act_base, const float* targets,
-                                                     float* seed_base, float* loss_out, int32_t B) {
-  __shared__ float red[1024];
-  __shared__ float piece[kSoftmaxMaxPieces];
-  __shared__ float bcast[2];
-  const int tid = threadIdx.x;
-  const int b = blockIdx.x;
-  targets += static_cast<int64_t>(b) * n;
-  loss_out += b;
-  auto at = [&](int k) { return static_cast<int64_t>(ids[k]) * B + b; };
-  const float* act = act_base;
-  float* seed_field = seed_base;
-  // 1. max by a '>' scan from -inf (NaN is never taken), then a tree.
-  float m = -__builtin_huge_valf();
-  for (int k = tid; k < n; k += blockDim.x) {
-    const float a = act[at(k)];
-    if (a > m) m = a;
+// The largest of a wave's values by a '>' scan (NaN is never taken).
+__device__ __forceinline__ float wave_peak(float m) {
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) {
+    const float o = __shfl_xor(m, w);
+    if (o > m) m = o;
   }
-  red[tid] = m;
-  __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if (tid < w && red[tid + w] > red[tid]) red[tid] = red[tid + w];
-    __syncthreads();
-  }
-  const float peak = red[0];
-  const int npieces = (n + kPiece - 1) / kPiece;
-  // 2. sum of exp(a - peak), piecewise.
-  for (int p = tid; p < npieces; p += blockDim.x) {
-    float s = 0.0f;
-    const int end = min(n, (p + 1) * kPiece);
-    for (int k = p * kPiece; k < end; ++k) s = s + px::expf_(act[at(k)] - peak);
-    piece[p] = s;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    float s = 0.0f;
-    for (int p = 0; p < npieces; ++p) s = s + piece[p];
-    bcast[0] = s;
-    bcast[1] = px::logf_(s);
-  }
-  __syncthreads();
-  const float total = bcast[0], log_sum = bcast[1];
-  // 3. seeds and the piecewise loss fold.
-  for (int p = tid; p < npieces; p += blockDim.x) {
-    float s = 0.0f;
-    const int end = min(n, (p + 1) * kPiece);
-    for (int k = p * kPiece; k < end; ++k) {
-      const float z = act[at(k)] - peak;
-      const float t = targets[k];
-      seed_field[at(k)] = px::expf_(z) / total - t;
-      s = s + t * (log_sum - z);
-    }
-    piece[p] = s;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    float s = 0.0f;
-    for (int p = 0; p < npieces; ++p) s = s + piece[p];
-    *loss_out = 0.0f + s;
-  }
+  return m;
 }
 
+// Workgroup b is sample b: unit u at u * B + b, targets[b * n ..], loss_out[b].
+// n <= kSoftmaxOne; thread t holds outputs t, t + blockDim, ...
+__global__ __launch_bounds__(1024) void k_softmax_ce(int32_t n, const int32_t* ids, const float* act,
+                                                     const float* targets, float* seed, float* loss_out,
+                                                     int32_t B) {
+  __shared__ __align__(16) float rows[kSoftmaxOne / kPiece * kPieceStride];
+  __shared__ __align__(16) float piece[kSoftmaxOne / kPiece];
+  __shared__ float peaks[16];
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const int b = blockIdx.x;
+  const int npieces = (n + kPiece - 1) / kPiece;
+  int64_t at[kSoftmaxPer];
+  float a[kSoftmaxPer], t[kSoftmaxPer];
+#pragma unroll
+  for (int i = 0; i < kSoftmaxPer; ++i) {
+    const int k = tid + i * nt;
+    at[i] = k < n ? static_cast<int64_t>(ids[k]) * B + b : -1;
+    t[i] = k < n ? targets[static_cast<int64_t>(b) * n + k] : 0.0f;
+  }
+  float m = -__builtin_huge_valf();
+#pragma unroll
+  for (int i = 0; i < kSoftmaxPer; ++i) {
+    a[i] = at[i] >= 0 ? act[at[i]] : -__builtin_huge_valf();
+    if (a[i] > m) m = a[i];
+  }
+  m = wave_peak(m);
+  if ((tid & 63) == 0) peaks[tid >> 6] = m;
+  __syncthreads();
+  float peak = peaks[0];
+  for (int w = 1; w < nt >> 6; ++w)
+    if (peaks[w] > peak) peak = peaks[w];
+  // 1. exp(a - peak), summed piece by piece.
+#pragma unroll
+  for (int i = 0; i < kSoftmaxPer; ++i) {
+    const int k = tid + i * nt;
+    a[i] = a[i] - peak;
+    if (at[i] >= 0) rows[k / kPiece * kPieceStride + k % kPiece] = px::expf_(a[i]);
+  }
+  __syncthreads();
+  if (tid < npieces) piece[tid] = fold_in_order(rows + tid * kPieceStride, min(kPiece, n - tid * kPiece), 0.0f);
+  __syncthreads();
+  const float total = fold_in_order(piece, npieces, 0.0f);
+  const float log_sum = px::logf_(total);
+  // 2. Seeds, and the loss terms in the exponentials' place (each thread
+  // replaces its own; the pieces were folded before the last barrier).
+#pragma unroll
+  for (int i = 0; i < kSoftmaxPer; ++i) {
+    if (at[i] < 0) continue;
+    const int k = tid + i * nt;
+    float* row = rows + k / kPiece * kPieceStride + k % kPiece;
+    seed[at[i]] = *row / total - t[i];
+    *row = t[i] * (log_sum - a[i]);
+  }
+  __syncthreads();
+  if (tid < npieces) piece[tid] = fold_in_order(rows + tid * kPieceStride, min(kPiece, n - tid * kPiece), 0.0f);
+  __syncthreads();
+  if (tid == 0) loss_out[b] = 0.0f + fold_in_order(piece, npieces, 0.0f);
+}
+
+// The many-output form: a workgroup per (sample, piece), samples from b0;
+// `peaks`, `sums` and `losses` hold np values per sample.
+struct SoftmaxAt {
+  int b, piece, k;  // sample, piece, this thread's output
+  __device__ __forceinline__ SoftmaxAt(int np, int b0)
+      : b(b0 + static_cast<int>(blockIdx.x / np)), piece(static_cast<int>(blockIdx.x % np)),
+        k(piece * kPiece + static_cast<int>(threadIdx.x)) {}
+  __device__ __forceinline__ int64_t row(int np) const { return static_cast<int64_t>(b) * np; }
+};
+
+__global__ __launch_bounds__(kPiece) void k_softmax_max(int32_t n, int32_t np, int32_t b0, const int32_t* ids,
+                                                        const float* act, float* peaks, int32_t B) {
+  __shared__ float wave[kPiece / 64];
+  const SoftmaxAt c(np, b0);
+  float m = c.k < n ? act[static_cast<int64_t>(ids[c.k]) * B + c.b] : -__builtin_huge_valf();
+  if (!(m > -__builtin_huge_valf())) m = -__builtin_huge_valf();  // (NaN is never taken)
+  m = wave_peak(m);
+  if ((threadIdx.x & 63) == 0) wave[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < kPiece / 64; ++w)
+    if (wave[w] > m) m = wave[w];
+  peaks[c.row(np) + c.piece] = m;
+}
+
+// The largest of a sample's np piece maxima, on every thread.
+__device__ __forceinline__ float softmax_peak(const float* peaks, int np, float* wave) {
+  float m = -__builtin_huge_valf();
+  for (int p = threadIdx.x; p < np; p += kPiece)
+    if (peaks[p] > m) m = peaks[p];
+  m = wave_peak(m);
+  if ((threadIdx.x & 63) == 0) wave[threadIdx.x >> 6] = m;
+  __syncthreads();
+  m = wave[0];
+  for (int w = 1; w < kPiece / 64; ++w)
+    if (wave[w] > m) m = wave[w];
+  return m;
+}
+
+__global__ __launch_bounds__(kPiece) void k_softmax_sum(int32_t n, int32_t np, int32_t b0, const int32_t* ids,
+                                                        const float* act, const float* peaks, float* sums,
+                                                        int32_t B) {
+  __shared__ __align__(16) float ex[kPiece];
+  __shared__ float wave[kPiece / 64];
+  const SoftmaxAt c(np, b0);
+  const float a = c.k < n ? act[static_cast<int64_t>(ids[c.k]) * B + c.b] : 0.0f;
+  ex[threadIdx.x] = px::expf_(a - softmax_peak(peaks + c.row(np), np, wave));
+  __syncthreads();
+  if (threadIdx.x == 0) sums[c.row(np) + c.piece] = fold_in_order(ex, min(kPiece, n - c.piece * kPiece), 0.0f);
+}
+
+__global__ __launch_bounds__(kPiece) void k_softmax_seed(int32_t n, int32_t np, int32_t b0, const int32_t* ids,
+                                                         const float* act, const float* targets,
+                                                         const float* peaks, const float* sums, float* seed,
+                                                         float* losses, int32_t B) {
+  __shared__ __align__(16) float part[kSoftmaxMaxPieces];
+  __shared__ __align__(16) float terms[kPiece];
+  __shared__ float wave[kPiece / 64];
+  __shared__ float whole;
+  const SoftmaxAt c(np, b0);
+  const int64_t at = c.k < n ? static_cast<int64_t>(ids[c.k]) * B + c.b : 0;
+  const float a = c.k < n ? act[at] : 0.0f;
+  const float t = c.k < n ? targets[static_cast<int64_t>(c.b) * n + c.k] : 0.0f;
+  for (int p = threadIdx.x; p < np; p += kPiece) part[p] = sums[c.row(np) + p];
+  const float z = a - softmax_peak(peaks + c.row(np), np, wave);  // (its barrier also closes the staging of part)
+  if (threadIdx.x == 0) whole = fold_in_order(part, np, 0.0f);
+  __syncthreads();
+  const float total = whole, log_sum = px::logf_(total);
+  if (c.k < n) seed[at] = px::expf_(z) / total - t;
+  terms[threadIdx.x] = t * (log_sum - z);
+  __syncthreads();
+  if (threadIdx.x == 0) losses[c.row(np) + c.piece] = fold_in_order(terms, min(kPiece, n - c.piece * kPiece), 0.0f);
+}
 
 __global__ void k_philox(int64_t n, const uint64_t* seeds, const uint64_t* ctrs, uint32_t* out) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1550,7 +1657,7 @@ extern "C" {
 
 const char* plx_last_error(void) { return plx_detail::g_last_error.c_str(); }
 
-int32_t plx_abi_version(void) { return 28; }
+int32_t plx_abi_version(void) { return 29; }
 
 int plx_struct_sizes(int64_t* out, int32_t n) {
   const int64_t sizes[20] = {
@@ -1765,15 +1872,33 @@ int plx_loss_elementwise(int32_t n_out, const int32_t* output_ids, const float* 
 }
 
 int plx_loss_softmax_ce(int32_t n_out, const int32_t* output_ids, const float* act,
-                        const float* targets, float* seed_field, float* loss_out,
-                        void* stream) {
-  if (n_out < 0) return fail(PLX_ERR_INVALID, "plx_loss_softmax_ce: negative n_out");
+                        const float* targets, float* seed_field, float* partials, float* losses,
+                        int32_t batch, void* stream) {
+  if (n_out < 0 || batch < 1) return fail(PLX_ERR_INVALID, "plx_loss_softmax_ce: bad size");
   if (n_out > kSoftmaxMaxPieces * kPiece)
     return fail(PLX_ERR_UNSUPPORTED, "plx_loss_softmax_ce: more than 262144 outputs");
-  if (!loss_out || (n_out > 0 && (!output_ids || !act || !targets || !seed_field)))
+  if (!losses || (n_out > 0 && (!output_ids || !act || !targets || !seed_field)))
     return fail(PLX_ERR_INVALID, "plx_loss_softmax_ce: null pointer");
-  k_softmax_ce<<<1, 1024, 0, static_cast<hipStream_t>(stream)>>>(n_out, output_ids, act,
-                                                                  targets, seed_field, loss_out, 1);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (n_out <= kSoftmaxOne) {
+    const unsigned block = n_out >= 1024 ? 1024u : (n_out > 0 ? static_cast<unsigned>((n_out + 63) / 64 * 64) : 64u);
+    k_softmax_ce<<<batch, block, 0, s>>>(n_out, output_ids, act, targets, seed_field, losses, batch);
+    return check_launch("plx_loss_softmax_ce");
+  }
+  if (!partials) return fail(PLX_ERR_INVALID, "plx_loss_softmax_ce: more than PLX_SOFTMAX_ONE outputs need partials");
+  const int np = (n_out + kPiece - 1) / kPiece;
+  float* peaks = partials;
+  float* sums = peaks + static_cast<int64_t>(np) * batch;
+  float* piece_losses = sums + static_cast<int64_t>(np) * batch;
+  const int chunk = (1 << 22) / np;  // samples per launch (a grid of at most 2^30 lanes)
+  for (int b0 = 0; b0 < batch; b0 += chunk) {
+    const unsigned grid = static_cast<unsigned>(np) * static_cast<unsigned>(batch - b0 < chunk ? batch - b0 : chunk);
+    k_softmax_max<<<grid, kPiece, 0, s>>>(n_out, np, b0, output_ids, act, peaks, batch);
+    k_softmax_sum<<<grid, kPiece, 0, s>>>(n_out, np, b0, output_ids, act, peaks, sums, batch);
+    k_softmax_seed<<<grid, kPiece, 0, s>>>(n_out, np, b0, output_ids, act, targets, peaks, sums, seed_field,
+                                           piece_losses, batch);
+  }
+  k_fold_sums<<<batch, 1024, 0, s>>>(np, piece_losses, losses);
   return check_launch("plx_loss_softmax_ce");
 }
 
@@ -1981,19 +2106,6 @@ int plx_loss_elementwise_batch(int32_t n_out, const int32_t* output_ids, const f
   }
   k_fold_sums<<<batch, 1024, 0, s>>>(npieces, partials, losses);
   return check_launch("plx_loss_elementwise_batch");
-}
-
-int plx_loss_softmax_ce_batch(int32_t n_out, const int32_t* output_ids, const float* act,
-                              const float* targets, float* seed_field, float* losses,
-                              int32_t batch, void* stream) {
-  if (n_out < 0 || batch < 1) return fail(PLX_ERR_INVALID, "plx_loss_softmax_ce_batch: bad size");
-  if (n_out > kSoftmaxMaxPieces * kPiece)
-    return fail(PLX_ERR_UNSUPPORTED, "plx_loss_softmax_ce_batch: more than 262144 outputs");
-  if (!losses || (n_out > 0 && (!output_ids || !act || !targets || !seed_field)))
-    return fail(PLX_ERR_INVALID, "plx_loss_softmax_ce_batch: null pointer");
-  k_softmax_ce<<<batch, 1024, 0, static_cast<hipStream_t>(stream)>>>(n_out, output_ids, act, targets,
-                                                                      seed_field, losses, batch);
-  return check_launch("plx_loss_softmax_ce_batch");
 }
 
 int plx_batch_mean(int32_t batch, const float* losses, float* out, void* stream) {

@@ -112,6 +112,13 @@ def _stream(device: torch.device) -> int:
     return int(torch.cuda.current_stream(device).cuda_stream)
 
 
+def softmax_partials(n_out: int, batch: int, device: torch.device) -> torch.Tensor | None:
+    """plx_loss_softmax_ce's scratch (None where it runs in one workgroup)."""
+    if n_out <= _lib.PLX_SOFTMAX_ONE:
+        return None
+    return torch.empty(3 * batch * -(-n_out // 256), dtype=torch.float32, device=device)
+
+
 class StepFn:
     """The callable ``make_step`` returns."""
 
@@ -664,6 +671,7 @@ class StepFn:
         lp = plan.loss
         seed = units[lp.seed_field]
         if lp.kind == "softmax":
+            parts = softmax_partials(n_out, 1, dev)
             _lib.check(
                 lib.plx_loss_softmax_ce(
                     n_out,
@@ -671,7 +679,9 @@ class StepFn:
                     units[ACTIVATION.name].data_ptr(),
                     t.data_ptr(),
                     seed.data_ptr(),
+                    None if parts is None else parts.data_ptr(),
                     loss.data_ptr(),
+                    1,
                     stream,
                 ),
                 "plx_loss_softmax_ce",
