@@ -1056,6 +1056,21 @@ PLX_EXPORT int plx_cold_slots(int64_t n, const int32_t* n_dev, const int32_t* co
 PLX_EXPORT int plx_copy_to_slots(int64_t n, const int32_t* n_dev, const int32_t* pos, const int32_t* slot,
                                  const void* src, void* dst, int64_t dst_len, int32_t bytes, void* stream);
 
+/* Positions [0, n) of a bucket's slab (at most *n_dev when given) back into
+ * their logical slots: dst[j][slot[p]] = src[j][p] for each of ncols columns
+ * of bytes[j] (1 or 4) bytes (src, dst, bytes: host arrays); positions whose
+ * slot lies outside [0, limit) are skipped. Column `stamped` (-1: none: a step
+ * count kept as one number while edges live) is not copied at the positions
+ * below `live` whose dead byte is 0. slot and the columns hold whole quads (n
+ * rounded up to 4). */
+#define PLX_MAX_SLOT_COLS 8
+PLX_EXPORT int plx_write_slots(int64_t n, const int32_t* n_dev, const int32_t* slot, int64_t limit, int32_t ncols,
+                               const void* const* src, void* const* dst, const int32_t* bytes, int32_t stamped,
+                               const uint8_t* dead, int64_t live, void* stream);
+
+/* out[i] = value for the i in [0, n) whose dead byte is 0. */
+PLX_EXPORT int plx_fill_live(int64_t n, const uint8_t* dead, float value, float* out, void* stream);
+
 /* One side of a merge: n elements whose ids (in [0, id_limit)) are listed
  * in ascending (key1[id], key2[id]) order, keys compared as uint32; key2
  * null means the id itself. map (optional, id_limit entries) receives each

@@ -393,12 +393,6 @@ class ChurnArena(Arena):
         """No source-value tables: units keep the caller's ids."""
         return 0, 0
 
-    def wrote(self, columns=None) -> None:
-        if columns is None or self._written is None:
-            self._written = None
-        else:
-            self._written |= {c for c in columns if c is not None}
-
     def write_logical(self, conns: tuple[Columns, ...]) -> None:
         """Scatter the live part of every bucket back into its logical slots
         (the slots dead at layout time were never written by the step): the
@@ -408,28 +402,9 @@ class ChurnArena(Arena):
         if written is not None and written <= {DEAD.name, self.t_name}:
             self._write_kills(conns, written)
             return
-        from plastax_amd.grow import Kernels
-
-        k = Kernels(self.device, int(torch.cuda.current_stream(self.device).cuda_stream))
         for b, bucket in enumerate(conns):
-            base, live, cap = self.bases[b], self.lives[b], self.caps[b]
-            if live == 0:
-                continue
             # positions [0, live count) to their logical slots (the count on the device)
-            every = k.iota(live)
-            for name, col in bucket.items():
-                if written is not None and name not in written:
-                    continue
-                vals = self.cols[name][base : base + live]
-                if name == self.t_name and self.t_now and self.t_now[b] is not None:
-                    # Live edges hold the bucket's count; an edge tombstoned
-                    # since the layout keeps the count stamped at its kill.
-                    vals = torch.where(self.cols[DEAD.name][base : base + live] != 0, vals,
-                                       torch.tensor(self.t_now[b], dtype=vals.dtype, device=vals.device))
-                vals = vals.contiguous()
-                _lib.check(k.lib.plx_copy_to_slots(live, self.live_dev[b].data_ptr(), every.data_ptr(),
-                                                   self.slot[base:].data_ptr(), vals.data_ptr(), col.data_ptr(), cap,
-                                                   col.element_size(), k.s), "plx_copy_to_slots")
+            self._write_bucket(b, bucket, written, self.lives[b], n_dev=self.live_dev[b])
 
 
 def _side(side, n: int, limit: int, ids: torch.Tensor, key1: torch.Tensor, key2: torch.Tensor | None,

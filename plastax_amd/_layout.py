@@ -48,6 +48,7 @@ as one contiguous slice.
 
 from __future__ import annotations
 
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -317,6 +318,7 @@ class Arena:
         # Adam's step count when every live edge of a bucket holds the same
         # one (per bucket; None: the per-edge column is authoritative).
         self.t_name: str | None = None
+        self._written: set | None = set()  # columns written since the logical view was in step (None: any)
         self.t_now: list[float | None] = []
         for b in range(nb):
             base, cap = self.bases[b], caps[b]
@@ -537,7 +539,56 @@ class Arena:
         )
 
     def write_logical(self, conns: tuple[Columns, ...]) -> None:
-        """Scatter the physical columns back into the logical buckets (unit
+        """The columns a step wrote since the last such copy, scattered back
+        into the logical buckets (the logical view's other columns are in
+        step: a layout's edges, ids and slots never change in place)."""
+        written, self._written = self._written, set()
+        if self.device.type != "cuda":
+            self._write_logical_host(conns)
+            return
+        for b, bucket in enumerate(conns):
+            # What a step writes lies among the positions live at layout time;
+            # a caller that names no columns may have written any.
+            self._write_bucket(b, bucket, written, self.caps[b] if written is None else self.lives[b])
+
+    def _write_bucket(self, b: int, bucket: Columns, written: set | None, n: int,
+                      n_dev: torch.Tensor | None = None) -> None:
+        """The ``written`` columns (None: any but the ids) of positions
+        [0, n) of bucket b (at most ``n_dev``) into its logical slots."""
+        from plastax_amd import _lib
+
+        names = [c for c in bucket if c not in (FROM_ID.name, TO_ID.name) and (written is None or c in written)]
+        if n == 0 or not names:
+            return
+        lib = _lib.load()
+        stream = int(torch.cuda.current_stream(self.device).cuda_stream)
+        base, cap = self.bases[b], self.caps[b]
+        # The bucket's shared step count: live edges hold it; an edge
+        # tombstoned since the layout keeps the count stamped at its kill,
+        # scattered back with its tombstone.
+        shared = self.t_name if self.t_name in names and self.t_now and self.t_now[b] is not None else None
+        if shared is not None and DEAD.name not in names:
+            names.remove(shared)
+        for c in [c for c in names if self.cols[c].element_size() not in (1, 4)]:
+            names.remove(c)
+            bucket[c][self.slot[base : base + n].long()] = self.cols[c][base : base + n]
+        for c0 in range(0, len(names), _lib.PLX_MAX_SLOT_COLS):
+            part = names[c0 : c0 + _lib.PLX_MAX_SLOT_COLS]
+            cols = [self.cols[c] for c in part]
+            src = (ctypes.c_void_p * len(part))(*[c.data_ptr() + base * c.element_size() for c in cols])
+            dst = (ctypes.c_void_p * len(part))(*[bucket[c].data_ptr() for c in part])
+            size = (ctypes.c_int32 * len(part))(*[c.element_size() for c in cols])
+            _lib.check(lib.plx_write_slots(
+                n, None if n_dev is None else n_dev.data_ptr(), self.slot.data_ptr() + 4 * base, cap, len(part),
+                ctypes.addressof(src), ctypes.addressof(dst), ctypes.addressof(size),
+                part.index(shared) if shared in part else -1, self.cols[DEAD.name].data_ptr() + base, self.lives[b],
+                stream), "plx_write_slots")
+        if shared is not None:
+            _lib.check(lib.plx_fill_live(cap, bucket[DEAD.name].data_ptr(), float(self.t_now[b]),
+                                         bucket[shared].data_ptr(), stream), "plx_fill_live")
+
+    def _write_logical_host(self, conns: tuple[Columns, ...]) -> None:
+        """write_logical of an arena laid out on the CPU: every column (unit
         ids mapped back to the caller's numbering)."""
         for b, bucket in enumerate(conns):
             base, cap = self.bases[b], self.caps[b]
@@ -548,15 +599,17 @@ class Arena:
                     vals = self.uperm_t[vals.long()].to(col.dtype)
                 col[idx] = vals
                 if name == self.t_name and self.t_now and self.t_now[b] is not None:
-                    # Live edges hold the bucket's count; an edge tombstoned
-                    # since the layout keeps the count stamped at its kill.
                     live = slice(base, base + self.lives[b])
                     col[idx[: self.lives[b]]] = torch.where(self.cols[DEAD.name][live] != 0, self.cols[name][live],
                                                             self.t_now[b])
 
     def wrote(self, columns: Any = None) -> None:
-        """A step wrote ``columns`` (None: any) of this arena; write_logical
-        copies every column back regardless."""
+        """A step wrote ``columns`` (None: any) of this arena: write_logical
+        copies them back."""
+        if columns is None or self._written is None:
+            self._written = None
+        else:
+            self._written |= {c for c in columns if c is not None}
 
     def init_uniform_t(self, t_name: str) -> None:
         """Adam's per-edge step count: where every live edge of a bucket holds

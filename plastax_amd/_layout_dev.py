@@ -134,6 +134,7 @@ class DeviceArena(Arena):
         self.prune_sink = None
         self.t_name = None
         self.t_now = []
+        self._written = set()
         nbits = _bits(n)
         for b, bucket in enumerate(conns):
             base, cap = self.bases[b], caps[b]

@@ -37,7 +37,7 @@ from plastax_amd import _layout, _lib
 from plastax_amd._expr import UnsupportedPolicyError
 from plastax_amd._layout import Arena
 from plastax_amd._plan import Plan, program_struct
-from plastax_amd._types import ACTIVATION
+from plastax_amd._types import ACTIVATION, WEIGHT
 from plastax_amd.state import NetworkState, NetworkStatic
 from plastax_amd.step import StepFn, StepInputs, StepResult, _stream, softmax_partials
 from plastax_amd.traits import Reduction, batch_written_reduction
@@ -376,7 +376,7 @@ class BatchedStepFn(StepFn):
         if up is not None:
             for b in range(arena.num_buckets):
                 self._update_batch(plan, arena, ub, consts, b, stream)
-            state._mark_ahead()
+            state._mark_ahead({WEIGHT.name, *up.state_columns()})
         if plan.update_generic:
             self._mean_of_writes(arena, ub, g, stream)
             state._mark_ahead()

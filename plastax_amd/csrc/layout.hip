@@ -238,6 +238,86 @@ __global__ void k_copy_to_slots(int64_t n, const int32_t* n_dev, const int32_t* 
   else static_cast<uint32_t*>(dst)[s] = static_cast<const uint32_t*>(src)[p];
 }
 
+// Positions [0, n) of a bucket's slab back into their logical slots, every
+// column of the launch in one pass over `slot`, four positions per lane
+// (V = 4: 16-byte loads; V = 1 where a column is not aligned for them). The
+// stores are 4-byte scatters, which bound the pass: a source's slots are
+// contiguous and its edges ascend by destination, so neighbouring positions'
+// stores fall into lines that later positions complete, provided one L2 sees
+// them all. Workgroup w runs on XCD w % 8: each XCD takes one contiguous
+// eighth of the positions, its workgroups in order.
+constexpr int kSlotBlock = 256;
+struct SlotCols {
+  const void* src[PLX_MAX_SLOT_COLS];
+  void* dst[PLX_MAX_SLOT_COLS];
+  int32_t bytes[PLX_MAX_SLOT_COLS];
+  int32_t n, stamped;
+};
+
+template <int V>
+__global__ __launch_bounds__(kSlotBlock) void k_write_slots(int64_t n_max, const int32_t* n_dev, const int32_t* slot,
+                                                            int64_t limit, SlotCols c, const uint8_t* dead,
+                                                            int64_t live) {
+  int64_t n = n_max;
+  if (n_dev) {
+    const int64_t m = *n_dev;
+    n = m < 0 ? 0 : (m < n ? m : n);
+  }
+  constexpr int kSpan = V * kSlotBlock;
+  const int64_t chunks = (n + kSpan - 1) / kSpan;
+  const int x = blockIdx.x & 7;
+  const int64_t c1 = chunks * (x + 1) / 8;
+  for (int64_t k = chunks * x / 8 + (blockIdx.x >> 3); k < c1; k += gridDim.x >> 3) {
+    const int64_t p = k * kSpan + V * static_cast<int64_t>(threadIdx.x);
+    if (p >= n) continue;
+    int32_t at[V];
+    if (V == 4) {  // (a slab is padded to whole quads)
+      const int4 q = *reinterpret_cast<const int4*>(slot + p);
+      at[0] = q.x, at[V > 1 ? 1 : 0] = q.y, at[V > 2 ? 2 : 0] = q.z, at[V > 3 ? 3 : 0] = q.w;
+    } else {
+      at[0] = slot[p];
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      if (p + i >= n || at[i] >= limit) at[i] = -1;
+    for (int j = 0; j < c.n; ++j) {
+      if (c.bytes[j] == 1) {
+        const uint8_t* s = static_cast<const uint8_t*>(c.src[j]) + p;
+        uint8_t v[V];
+        if (V == 4) {
+          const uint32_t q = *reinterpret_cast<const uint32_t*>(s);
+#pragma unroll
+          for (int i = 0; i < V; ++i) v[i] = static_cast<uint8_t>(q >> (8 * i));
+        } else {
+          v[0] = s[0];
+        }
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+          if (at[i] >= 0) static_cast<uint8_t*>(c.dst[j])[at[i]] = v[i];
+        continue;
+      }
+      const uint32_t* s = static_cast<const uint32_t*>(c.src[j]) + p;
+      uint32_t v[V];
+      if (V == 4) {
+        const uint4 q = *reinterpret_cast<const uint4*>(s);
+        v[0] = q.x, v[V > 1 ? 1 : 0] = q.y, v[V > 2 ? 2 : 0] = q.z, v[V > 3 ? 3 : 0] = q.w;
+      } else {
+        v[0] = s[0];
+      }
+#pragma unroll
+      for (int i = 0; i < V; ++i)
+        if (at[i] >= 0 && (j != c.stamped || p + i >= live || dead[p + i] != 0))
+          static_cast<uint32_t*>(c.dst[j])[at[i]] = v[i];
+    }
+  }
+}
+
+__global__ void k_fill_live(int64_t n, const uint8_t* dead, float value, float* out) {
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+    if (!dead[i]) out[i] = value;
+}
+
 // The (key1, key2) of id `id` of a merge side, as one 64-bit unsigned key;
 // ids are clamped into [0, id_limit) for the reads.
 __device__ __forceinline__ uint64_t merge_key(const plx_merge_side& s, int64_t id) {
@@ -622,6 +702,52 @@ int plx_copy_to_slots(int64_t n, const int32_t* n_dev, const int32_t* pos, const
   hipLaunchKernelGGL(k_copy_to_slots, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), n, n_dev, pos, slot, src, dst, dst_len, bytes);
   return check_launch("plx_copy_to_slots");
+}
+
+int plx_write_slots(int64_t n, const int32_t* n_dev, const int32_t* slot, int64_t limit, int32_t ncols,
+                    const void* const* src, void* const* dst, const int32_t* bytes, int32_t stamped,
+                    const uint8_t* dead, int64_t live, void* stream) {
+  if (n < 0 || limit < 0 || ncols < 0 || ncols > PLX_MAX_SLOT_COLS || stamped >= ncols)
+    return fail(PLX_ERR_INVALID, "plx_write_slots: bad size");
+  if (n == 0 || ncols == 0) return PLX_OK;
+  if (!slot || !src || !dst || !bytes || (stamped >= 0 && !dead))
+    return fail(PLX_ERR_INVALID, "plx_write_slots: null pointer");
+  SlotCols c{};
+  c.n = ncols;
+  c.stamped = stamped < 0 ? -1 : stamped;
+  auto aligned = [](const void* p, int b) { return reinterpret_cast<uintptr_t>(p) % b == 0; };
+  bool quads = aligned(slot, 16);
+  for (int32_t j = 0; j < ncols; ++j) {
+    if (!src[j] || !dst[j]) return fail(PLX_ERR_INVALID, "plx_write_slots: null column");
+    if (bytes[j] != 1 && bytes[j] != 4) return fail(PLX_ERR_INVALID, "plx_write_slots: bytes must be 1 or 4");
+    if (j == stamped && bytes[j] != 4)
+      return fail(PLX_ERR_INVALID, "plx_write_slots: the stamped column holds 4-byte values");
+    quads = quads && aligned(src[j], 4 * bytes[j]);
+    c.src[j] = src[j];
+    c.dst[j] = dst[j];
+    c.bytes[j] = bytes[j];
+  }
+  // A multiple of eight workgroups (one share per XCD), eight per CU at most.
+  const int64_t span = (quads ? 4 : 1) * kSlotBlock;
+  const int64_t want = ((n + span - 1) / span + 7) / 8 * 8;
+  const int64_t most = static_cast<int64_t>(plx_detail::cu_count()) * 8;
+  const unsigned grid = static_cast<unsigned>(want < most ? want : most);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (quads)
+    hipLaunchKernelGGL(k_write_slots<4>, dim3(grid), dim3(kSlotBlock), 0, s, n, n_dev, slot, limit, c, dead, live);
+  else
+    hipLaunchKernelGGL(k_write_slots<1>, dim3(grid), dim3(kSlotBlock), 0, s, n, n_dev, slot, limit, c, dead, live);
+  return check_launch("plx_write_slots");
+}
+
+int plx_fill_live(int64_t n, const uint8_t* dead, float value, float* out, void* stream) {
+  if (n < 0) return fail(PLX_ERR_INVALID, "plx_fill_live: negative n");
+  if (n == 0) return PLX_OK;
+  if (!dead || !out) return fail(PLX_ERR_INVALID, "plx_fill_live: null pointer");
+  const int64_t want = (n + 255) / 256;
+  hipLaunchKernelGGL(k_fill_live, dim3(static_cast<unsigned>(want < 4096 ? want : 4096)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), n, dead, value, out);
+  return check_launch("plx_fill_live");
 }
 
 static bool merge_side_ok(const plx_merge_side& s) {

@@ -22,7 +22,7 @@ from plastax_amd import _lib
 from plastax_amd._expr import UnsupportedPolicyError
 from plastax_amd._layout import NSUPER, TILE, Arena
 from plastax_amd._plan import Plan, compile_plan, program_struct
-from plastax_amd._types import ACTIVATION, DEAD, Propagation
+from plastax_amd._types import ACTIVATION, DEAD, WEIGHT, Propagation
 from plastax_amd.fusion import PruneFusionPlan, PruneFusionRecord, plan_prune_fusion
 from plastax_amd.state import NetworkState, NetworkStatic
 
@@ -353,8 +353,10 @@ class StepFn:
         # bucket b's backward terms use its pre-update weights, and bucket b's
         # update needs only finalized grads (levels > b) and activations.
         self._backward_update(plan, arena, units, consts, fin_common, stream, g)
-        if plan.update is not None or plan.update_generic:
-            state._mark_ahead()
+        if plan.update is not None:
+            state._mark_ahead({WEIGHT.name, *plan.update.state_columns()})
+        if plan.update_generic:
+            state._mark_ahead({name for _, names in self._update_generic.passes for name in names})
 
         # Structural phases (phases.py:1245-1498, :4490-5203).
         if plan.prune_unit or plan.prune_conn or plan.add_unit or plan.add_conn is not None:
