@@ -1059,13 +1059,13 @@ PLX_EXPORT int plx_copy_to_slots(int64_t n, const int32_t* n_dev, const int32_t*
 /* Positions [0, n) of a bucket's slab (at most *n_dev when given) back into
  * their logical slots: dst[j][slot[p]] = src[j][p] for each of ncols columns
  * of bytes[j] (1 or 4) bytes (src, dst, bytes: host arrays); positions whose
- * slot lies outside [0, limit) are skipped. Column `stamped` (-1: none: a step
- * count kept as one number while edges live) is not copied at the positions
- * below `live` whose dead byte is 0. slot and the columns hold whole quads (n
- * rounded up to 4). */
+ * slot lies outside [0, limit) are skipped. A column whose bit is set in
+ * `killed` (DEAD; a step count kept as one number while edges live) is not
+ * copied at the positions below `live` whose dead byte is 0. slot and the
+ * columns hold whole quads (n rounded up to 4). */
 #define PLX_MAX_SLOT_COLS 8
 PLX_EXPORT int plx_write_slots(int64_t n, const int32_t* n_dev, const int32_t* slot, int64_t limit, int32_t ncols,
-                               const void* const* src, void* const* dst, const int32_t* bytes, int32_t stamped,
+                               const void* const* src, void* const* dst, const int32_t* bytes, uint32_t killed,
                                const uint8_t* dead, int64_t live, void* stream);
 
 /* out[i] = value for the i in [0, n) whose dead byte is 0. */

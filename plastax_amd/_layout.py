@@ -565,7 +565,8 @@ class Arena:
         base, cap = self.bases[b], self.caps[b]
         # The bucket's shared step count: live edges hold it; an edge
         # tombstoned since the layout keeps the count stamped at its kill,
-        # scattered back with its tombstone.
+        # scattered back with its tombstone (an edge live at layout time is
+        # live in the logical view until then).
         shared = self.t_name if self.t_name in names and self.t_now and self.t_now[b] is not None else None
         if shared is not None and DEAD.name not in names:
             names.remove(shared)
@@ -581,8 +582,8 @@ class Arena:
             _lib.check(lib.plx_write_slots(
                 n, None if n_dev is None else n_dev.data_ptr(), self.slot.data_ptr() + 4 * base, cap, len(part),
                 ctypes.addressof(src), ctypes.addressof(dst), ctypes.addressof(size),
-                part.index(shared) if shared in part else -1, self.cols[DEAD.name].data_ptr() + base, self.lives[b],
-                stream), "plx_write_slots")
+                sum(1 << j for j, c in enumerate(part) if c in (DEAD.name, shared)),
+                self.cols[DEAD.name].data_ptr() + base, self.lives[b], stream), "plx_write_slots")
         if shared is not None:
             _lib.check(lib.plx_fill_live(cap, bucket[DEAD.name].data_ptr(), float(self.t_now[b]),
                                          bucket[shared].data_ptr(), stream), "plx_fill_live")

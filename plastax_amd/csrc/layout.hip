@@ -251,7 +251,8 @@ struct SlotCols {
   const void* src[PLX_MAX_SLOT_COLS];
   void* dst[PLX_MAX_SLOT_COLS];
   int32_t bytes[PLX_MAX_SLOT_COLS];
-  int32_t n, stamped;
+  int32_t n;
+  uint32_t killed;  // bit j: column j only where the edge is dead
 };
 
 template <int V>
@@ -280,34 +281,32 @@ __global__ __launch_bounds__(kSlotBlock) void k_write_slots(int64_t n_max, const
 #pragma unroll
     for (int i = 0; i < V; ++i)
       if (p + i >= n || at[i] >= limit) at[i] = -1;
+    bool put[V];  // whether a column of killed edges is stored at the position
+#pragma unroll
+    for (int i = 0; i < V; ++i) put[i] = at[i] >= 0 && c.killed != 0 && (p + i >= live || dead[p + i] != 0);
     for (int j = 0; j < c.n; ++j) {
+      uint32_t v[V];
       if (c.bytes[j] == 1) {
         const uint8_t* s = static_cast<const uint8_t*>(c.src[j]) + p;
-        uint8_t v[V];
-        if (V == 4) {
-          const uint32_t q = *reinterpret_cast<const uint32_t*>(s);
+        const uint32_t q = V == 4 ? *reinterpret_cast<const uint32_t*>(s) : *s;
 #pragma unroll
-          for (int i = 0; i < V; ++i) v[i] = static_cast<uint8_t>(q >> (8 * i));
+        for (int i = 0; i < V; ++i) v[i] = (q >> (8 * i)) & 0xFFu;
+      } else {
+        const uint32_t* s = static_cast<const uint32_t*>(c.src[j]) + p;
+        if (V == 4) {
+          const uint4 q = *reinterpret_cast<const uint4*>(s);
+          v[0] = q.x, v[V > 1 ? 1 : 0] = q.y, v[V > 2 ? 2 : 0] = q.z, v[V > 3 ? 3 : 0] = q.w;
         } else {
           v[0] = s[0];
         }
-#pragma unroll
-        for (int i = 0; i < V; ++i)
-          if (at[i] >= 0) static_cast<uint8_t*>(c.dst[j])[at[i]] = v[i];
-        continue;
       }
-      const uint32_t* s = static_cast<const uint32_t*>(c.src[j]) + p;
-      uint32_t v[V];
-      if (V == 4) {
-        const uint4 q = *reinterpret_cast<const uint4*>(s);
-        v[0] = q.x, v[V > 1 ? 1 : 0] = q.y, v[V > 2 ? 2 : 0] = q.z, v[V > 3 ? 3 : 0] = q.w;
-      } else {
-        v[0] = s[0];
-      }
+      const bool some = (c.killed >> j) & 1u;
 #pragma unroll
-      for (int i = 0; i < V; ++i)
-        if (at[i] >= 0 && (j != c.stamped || p + i >= live || dead[p + i] != 0))
-          static_cast<uint32_t*>(c.dst[j])[at[i]] = v[i];
+      for (int i = 0; i < V; ++i) {
+        if (some ? !put[i] : at[i] < 0) continue;
+        if (c.bytes[j] == 1) static_cast<uint8_t*>(c.dst[j])[at[i]] = static_cast<uint8_t>(v[i]);
+        else static_cast<uint32_t*>(c.dst[j])[at[i]] = v[i];
+      }
     }
   }
 }
@@ -705,23 +704,21 @@ int plx_copy_to_slots(int64_t n, const int32_t* n_dev, const int32_t* pos, const
 }
 
 int plx_write_slots(int64_t n, const int32_t* n_dev, const int32_t* slot, int64_t limit, int32_t ncols,
-                    const void* const* src, void* const* dst, const int32_t* bytes, int32_t stamped,
+                    const void* const* src, void* const* dst, const int32_t* bytes, uint32_t killed,
                     const uint8_t* dead, int64_t live, void* stream) {
-  if (n < 0 || limit < 0 || ncols < 0 || ncols > PLX_MAX_SLOT_COLS || stamped >= ncols)
+  if (n < 0 || limit < 0 || ncols < 0 || ncols > PLX_MAX_SLOT_COLS)
     return fail(PLX_ERR_INVALID, "plx_write_slots: bad size");
   if (n == 0 || ncols == 0) return PLX_OK;
-  if (!slot || !src || !dst || !bytes || (stamped >= 0 && !dead))
+  if (!slot || !src || !dst || !bytes || (killed != 0 && !dead))
     return fail(PLX_ERR_INVALID, "plx_write_slots: null pointer");
   SlotCols c{};
   c.n = ncols;
-  c.stamped = stamped < 0 ? -1 : stamped;
+  c.killed = killed;
   auto aligned = [](const void* p, int b) { return reinterpret_cast<uintptr_t>(p) % b == 0; };
   bool quads = aligned(slot, 16);
   for (int32_t j = 0; j < ncols; ++j) {
     if (!src[j] || !dst[j]) return fail(PLX_ERR_INVALID, "plx_write_slots: null column");
     if (bytes[j] != 1 && bytes[j] != 4) return fail(PLX_ERR_INVALID, "plx_write_slots: bytes must be 1 or 4");
-    if (j == stamped && bytes[j] != 4)
-      return fail(PLX_ERR_INVALID, "plx_write_slots: the stamped column holds 4-byte values");
     quads = quads && aligned(src[j], 4 * bytes[j]);
     c.src[j] = src[j];
     c.dst[j] = dst[j];

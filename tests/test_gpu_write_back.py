@@ -1,7 +1,7 @@
 """Columns copied back into their logical slots (plx_write_slots,
 plx_fill_live) against numpy: counts around a workgroup's span, aligned and
 unaligned columns (the four- and one-position forms), byte and 4-byte columns,
-slots outside the bucket, a count on the device, the stamped column; and a
+slots outside the bucket, a count on the device, columns of killed edges; and a
 net's logical view read after every step and after several, with kills in
 between, against the oracle."""
 
@@ -38,7 +38,8 @@ def test_write_slots_matches_numpy(n: int, shift: int) -> None:
     dead = rng.integers(0, 2, shift + room).astype(np.uint8)
     live = max(n - 2, 0)
     count = max(n - 1, 1)
-    want = [np.zeros(limit, np.float32), np.zeros(limit, np.float32), np.zeros(limit, np.uint8)]
+    want = [np.zeros(limit, np.float32), np.zeros(limit, np.float32), np.zeros(limit, np.uint8),
+            np.zeros(limit, np.uint8)]
     for p in range(count):
         s = slot[shift + p]
         if s < 0:
@@ -47,16 +48,17 @@ def test_write_slots_matches_numpy(n: int, shift: int) -> None:
         want[2][s] = u[shift + p]
         if p >= live or dead[shift + p]:
             want[1][s] = g[shift + p]
+            want[3][s] = dead[shift + p]
     ts = [torch.from_numpy(v).to(DEV) for v in (slot, f, g, u, dead)]
     out = [torch.from_numpy(np.zeros_like(v)).to(DEV) for v in want]
     n_dev = torch.tensor([count], dtype=torch.int32, device=DEV)
     at = [t.data_ptr() + shift * t.element_size() for t in ts]
-    src = (ctypes.c_void_p * 3)(at[1], at[2], at[3])
-    dst = (ctypes.c_void_p * 3)(*[t.data_ptr() for t in out])
-    size = (ctypes.c_int32 * 3)(4, 4, 1)
+    src = (ctypes.c_void_p * 4)(at[1], at[2], at[3], at[4])
+    dst = (ctypes.c_void_p * 4)(*[t.data_ptr() for t in out])
+    size = (ctypes.c_int32 * 4)(4, 4, 1, 1)
     print(f"write slots n {n} shift {shift}", flush=True)
-    _lib.call("plx_write_slots", n, n_dev.data_ptr(), at[0], limit, 3, ctypes.addressof(src), ctypes.addressof(dst),
-              ctypes.addressof(size), 1, at[4], live, None)
+    _lib.call("plx_write_slots", n, n_dev.data_ptr(), at[0], limit, 4, ctypes.addressof(src), ctypes.addressof(dst),
+              ctypes.addressof(size), 0b1010, at[4], live, None)
     fill = torch.zeros(shift + room, device=DEV)
     _lib.call("plx_fill_live", n, at[4], 2.5, fill.data_ptr(), None)
     torch.cuda.synchronize()
