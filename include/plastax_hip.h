@@ -332,8 +332,10 @@ typedef struct plx_bwd_batch_desc {
   const int32_t* row_unit;
   const int32_t* row_ptr;
   const int32_t* dst;    /* [entries] TO_ID */
-  const float* weight;   /* [entries] WEIGHT */
-  const uint8_t* live;   /* [entries] 0: skipped (null: every entry live) */
+  const float* weight;   /* [entries] WEIGHT (with pos: [positions]) */
+  const uint8_t* live;   /* [entries] 0: skipped (null: every entry live; plx_backward_lists) */
+  const int32_t* pos;    /* [entries] the entry's position in weight and dead, or null: the entry itself */
+  const uint8_t* dead;   /* non-zero: skipped (null: none is; plx_backward_batch) */
   const float* g;        /* [num_units][B] the map's linear_input field */
   float* acc;            /* [num_units][B] carried accumulator, or null */
   plx_finalize fin;

@@ -214,6 +214,8 @@ class plx_bwd_batch_desc(ctypes.Structure):
         ("dst", c_vp),
         ("weight", c_vp),
         ("live", c_vp),
+        ("pos", c_vp),
+        ("dead", c_vp),
         ("g", c_vp),
         ("acc", c_vp),
         ("fin", plx_finalize),

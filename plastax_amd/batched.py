@@ -49,8 +49,7 @@ class BatchSources:
     """Per bucket, its backward rows (sources) and their out-edge lists in
     logical slot order: list entry j (``ptr[r] <= j < ptr[r+1]``) is physical
     position ``pos[j]``, whose TO_ID ``dst[j]`` is fixed with the layout; the
-    step gathers the entries' weights and liveness into ``weight`` / ``live``
-    (one wide gather), so the backward reads every list sequentially."""
+    backward reads its weight and tombstone at the position."""
 
     def __init__(self, nrows: int, rows: torch.Tensor, ptr: torch.Tensor, pos: torch.Tensor,
                  dst: torch.Tensor) -> None:
@@ -59,9 +58,6 @@ class BatchSources:
         self.ptr = ptr
         self.pos = pos
         self.dst = dst
-        n = int(pos.numel())
-        self.weight = torch.empty(n, dtype=torch.float32, device=pos.device)
-        self.live = torch.empty(n, dtype=torch.uint8, device=pos.device)
 
 
 def batch_sources(arena: Arena, b: int) -> BatchSources:
@@ -335,8 +331,11 @@ class BatchedStepFn(StepFn):
                 d.row_unit = rows.data_ptr()
                 d.row_ptr = ptr.data_ptr()
                 d.dst = lists.dst.data_ptr()
-                d.weight = lists.weight.data_ptr()
-                d.live = lists.live.data_ptr()
+                # This step's (pre-update) weights and tombstones, read at the
+                # entries' positions.
+                d.pos = lists.pos.data_ptr()
+                d.weight = arena.cols["weight"].data_ptr()
+                d.dead = arena.cols["dead"].data_ptr() if arena.dead_in_rows else None
                 d.g = bp.gathered(ub, ACTIVATION.name).data_ptr()
                 d.map = bp.map_struct()
                 d.acc = bacc.data_ptr() if bacc is not None else None
@@ -354,13 +353,6 @@ class BatchedStepFn(StepFn):
                 run(top.rows, top.nrows, zeros, none, nb)
             for b in range(nb - 1, 0, -1):
                 lists = batch_sources(arena, b)
-                # This step's (pre-update) weights and tombstones, in slot order.
-                _lib.check(
-                    lib.plx_gather_edges(lists.pos.numel(), lists.pos.data_ptr(), arena.cols["weight"].data_ptr(),
-                                         arena.cols["dead"].data_ptr(), lists.weight.data_ptr(),
-                                         lists.live.data_ptr(), stream),
-                    "plx_gather_edges",
-                )
                 run(lists.rows, lists.nrows, lists.ptr, lists, b)
 
         # update_unit, per sample (step.py:435-436), on the live units.

@@ -787,8 +787,7 @@ __global__ __launch_bounds__(kFinBlock) void k_finalize(plx_partials_desc d, int
 // Each lane folds its sample's terms in the streaming step's order.
 // ---------------------------------------------------------------------------
 constexpr int kBatchBlock = 256;
-constexpr int kBatchUnroll = 8;       // positions whose loads are in flight together (one wave per row)
-constexpr int kBatchUnrollWide = 16;  // the same for a 256-lane workgroup per row (levels of few, long rows)
+constexpr int kBatchUnroll = 8;  // unit rows loaded together by a wave of k_batch_rows
 
 // Combines a row's sum into acc and finalizes it for sample lane `idx`.
 template <int M>
@@ -803,183 +802,196 @@ __device__ __forceinline__ void finish_batch(float* acc, const plx_program& P, b
   }
 }
 
-template <int M>
-__global__ __launch_bounds__(kBatchBlock) void k_forward_batch(plx_forward_desc d, int32_t B) {
+// Entries of a batched row, the same for both directions: a forward row's
+// positions (source, weight, tombstone), a backward row's list entries
+// (destination; weight and tombstone of the position they name).
+__device__ __forceinline__ const int32_t* batch_other(const plx_forward_desc& d) { return d.src; }
+__device__ __forceinline__ const int32_t* batch_other(const plx_bwd_batch_desc& d) { return d.dst; }
+__device__ __forceinline__ int batch_pos(const plx_forward_desc&, int e) { return e; }
+__device__ __forceinline__ int batch_pos(const plx_bwd_batch_desc& d, int e) { return d.pos ? d.pos[e] : e; }
+__device__ __forceinline__ const uint8_t* batch_dead(const plx_forward_desc& d) { return d.dead; }
+__device__ __forceinline__ const uint8_t* batch_dead(const plx_bwd_batch_desc& d) { return d.dead; }
+__device__ __forceinline__ const float* batch_rows(const plx_forward_desc& d) { return d.x; }
+__device__ __forceinline__ const float* batch_rows(const plx_bwd_batch_desc& d) { return d.g; }
+
+// Levels of many rows: a wave per row and 64 V samples, V samples per lane (V =
+// 4: 16-byte loads, B a multiple of 4). It gathers a B-wide unit row per edge
+// from L2 and spends a product and an add per edge and sample; at 256 samples
+// both take 20 to 45 us per 1.7M edges, so neither may wait for the other and
+// nothing else may be issued per edge. The row ids come through the scalar
+// cache, eight at a time and two groups ahead, the unit rows one group ahead
+// of the fold, the weights 64 at a time, one per lane, handed out by readlane
+// (a backward entry's weight is read at its position, so no copy of the
+// weights in list order is made). PLAIN: both factors are loaded and no
+// tombstone is looked for, so an edge costs its products and adds alone. Mean
+// launch of the 784-4096-4096-10 net (321K and 1.7M edges, 256 samples):
+// forward 55.7 -> 51.1 us, backward 81.7 and a 16.5 us copy of the weights ->
+// 58.5; the two selects of a constant factor per edge and sample alone were 11
+// of the forward's (62.3 us with them). With one sample a lane, 1,003 and 777
+// rows at 70 samples: 15.9 -> 14.0.
+template <int V>
+struct BatchLane {
+  float v[V];
+};
+template <int V>
+__device__ __forceinline__ BatchLane<V> load_batch(const float* p) {
+  BatchLane<V> r;
+  if constexpr (V == 4) {
+    const float4 q = *reinterpret_cast<const float4*>(p);
+    r.v[0] = q.x, r.v[1] = q.y, r.v[2] = q.z, r.v[3] = q.w;
+  } else {
+    r.v[0] = *p;
+  }
+  return r;
+}
+
+template <int M, class D, int V, bool PLAIN>
+__device__ __forceinline__ void batch_row(const D& d, int B) {
+  constexpr int U = kBatchUnroll;
   const int r = blockIdx.x;
+  const int u = d.row_unit[r];
+  const int e0 = ld_uniform(d.row_ptr, r), e1 = ld_uniform(d.row_ptr, r + 1);
+  const bool fin = finalizes(d.fin, u);
+  const float ident = Mono<M>::id();
+  const int lane = static_cast<int>(threadIdx.x);
+  const int b = (static_cast<int>(blockIdx.y) * 64 + lane) * V;
+  const float* x = batch_rows(d) + (b < B ? b : B - V);  // every lane's loads stay in its row
+  const int32_t* other = batch_other(d);
+  const uint8_t* dead = batch_dead(d);
+  BatchLane<V> s;
+#pragma unroll
+  for (int j = 0; j < V; ++j) s.v[j] = ident;
+  if (e0 < e1) {
+    float w = 0.0f;  // entry c + lane of the chunk at c (past the row's end: its last one)
+    int gone = 0;
+    auto load_chunk = [&](int c) {
+      const int p = batch_pos(d, min(c + lane, e1 - 1));
+      w = d.weight[p];
+      if (!PLAIN) gone = dead ? dead[p] : 0;
+    };
+    int ia[U], ib[U];
+    BatchLane<V> ra[U], rb[U];
+    auto load_ids = [&](int(&id)[U], int e) {
+#pragma unroll
+      for (int k = 0; k < U; ++k) id[k] = ld_uniform(other, min(e + k, e1 - 1));
+    };
+    auto load_rows = [&](BatchLane<V>(&v)[U], const int(&id)[U]) {
+#pragma unroll
+      for (int k = 0; k < U; ++k) v[k] = load_batch<V>(x + static_cast<int64_t>(id[k]) * B);
+    };
+    load_chunk(e0);
+    load_ids(ia, e0);
+    load_rows(ra, ia);
+    load_ids(ib, e0 + U);
+    for (int c = e0; c < e1; c += 64) {
+      const float cw = w;
+      const int cg = gone;
+      if (c + 64 < e1) load_chunk(c + 64);
+      auto fold = [&](const BatchLane<V>(&v)[U], int e) {
+        auto one = [&](int k) {
+          const float wk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cw), e - c + k));
+          if (!PLAIN && __builtin_amdgcn_readlane(cg, e - c + k)) return;
+#pragma unroll
+          for (int j = 0; j < V; ++j)
+            s.v[j] = Mono<M>::op(s.v[j], PLAIN ? wk * v[k].v[j] : map_term(d.map, wk, v[k].v[j]));
+        };
+        if (e + U <= e1) {
+#pragma unroll
+          for (int k = 0; k < U; ++k) one(k);
+        } else {
+#pragma unroll
+          for (int k = 0; k < U; ++k)
+            if (e + k < e1) one(k);
+        }
+      };
+      const int ce = min(c + 64, e1);
+      for (int e = c; e < ce; e += 2 * U) {
+        if (e + U < e1) load_rows(rb, ib);
+        load_ids(ia, e + 2 * U);
+        fold(ra, e);
+        if (e + 2 * U < e1) load_rows(ra, ia);
+        load_ids(ib, e + 3 * U);
+        if (e + U < e1) fold(rb, e + U);
+      }
+    }
+  }
+  if (b < B)
+#pragma unroll
+    for (int j = 0; j < V; ++j) finish_batch<M>(d.acc, d.apply, fin, static_cast<int64_t>(u) * B + b + j, s.v[j]);
+}
+
+template <int M, class D, int V>
+__global__ __launch_bounds__(64) void k_batch_rows(D d, int32_t B) {
+  if (d.map.flags == 0 && !batch_dead(d))
+    batch_row<M, D, V, true>(d, B);
+  else
+    batch_row<M, D, V, false>(d, B);
+}
+
+// Levels of few rows: a workgroup per (row, kGroup samples), whose lanes form the terms of kGroupWin
+// entries side by side (a lane per sample and entry) into LDS, where a lane
+// per sample folds them in order while the next window's loads are in flight.
+// With a 256-lane workgroup per row such a level waited for one chain of id
+// and row loads per sixteen entries (ten rows of 410 edges, 256 samples:
+// 37.6 us, ten CUs busy; 11.0 in groups).
+constexpr int kGroup = 16;
+constexpr int kGroupWin = 256;
+constexpr int kGroupPer = kGroupWin * kGroup / kBatchBlock;  // entries per lane and window
+
+template <int M, class D>
+__global__ __launch_bounds__(kBatchBlock) void k_batch_groups(D d, int32_t B) {
+  __shared__ float term[2][kGroupWin][kGroup + 1];
+  const int r = blockIdx.x;
+  const int b0 = static_cast<int>(blockIdx.y) * kGroup;
   const int u = d.row_unit[r];
   const int e0 = d.row_ptr[r], e1 = d.row_ptr[r + 1];
-  const bool fin = finalizes(d.fin, u);
   const float ident = Mono<M>::id();
-  for (int b0 = 0; b0 < B; b0 += blockDim.x) {
-    const int b = b0 + static_cast<int>(threadIdx.x);
-    const int bl = b < B ? b : B - 1;  // every lane's loads stay in its row
-    float s = ident;
-    int e = e0;
-    for (; e + kBatchUnrollWide <= e1; e += kBatchUnrollWide) {
-      int sv[kBatchUnrollWide];
-      float wv[kBatchUnrollWide], xv[kBatchUnrollWide];
-      bool live[kBatchUnrollWide];
+  const int smp = static_cast<int>(threadIdx.x) % kGroup, sub = static_cast<int>(threadIdx.x) / kGroup;
+  const int b = b0 + smp, bl = b < B ? b : B - 1;  // every lane's loads stay in its row
+  const float* x = batch_rows(d);
+  const uint8_t* dead = batch_dead(d);
+  constexpr int kStep = kBatchBlock / kGroup;
+  float wv[kGroupPer], xv[kGroupPer];
+  bool use[kGroupPer];
+  auto load = [&](int w0) {
+    int o[kGroupPer];
 #pragma unroll
-      for (int k = 0; k < kBatchUnrollWide; ++k) {
-        sv[k] = d.src[e + k];
-        wv[k] = d.weight[e + k];
-        live[k] = d.dead ? d.dead[e + k] == 0 : true;
+    for (int i = 0; i < kGroupPer; ++i) {
+      const int e = w0 + sub + i * kStep;
+      const int at = min(e, e1 - 1);
+      o[i] = batch_other(d)[at];
+      const int p = batch_pos(d, at);
+      wv[i] = d.weight[p];
+      use[i] = e < e1 && !(dead && dead[p]);
+    }
+#pragma unroll
+    for (int i = 0; i < kGroupPer; ++i) xv[i] = x[static_cast<int64_t>(o[i]) * B + bl];
+  };
+  float s = ident;
+  if (e0 < e1) load(e0);
+  int par = 0;
+  for (int w0 = e0; w0 < e1; w0 += kGroupWin, par ^= 1) {
+#pragma unroll
+    for (int i = 0; i < kGroupPer; ++i)
+      term[par][sub + i * kStep][smp] = use[i] ? map_term(d.map, wv[i], xv[i]) : ident;
+    __syncthreads();
+    if (w0 + kGroupWin < e1) load(w0 + kGroupWin);
+    if (sub == 0) {
+      const int n = min(kGroupWin, e1 - w0);
+      int j = 0;
+      for (; j + 8 <= n; j += 8) {
+        float t[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) t[k] = term[par][j + k][smp];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s = Mono<M>::op(s, t[k]);
       }
-#pragma unroll
-      for (int k = 0; k < kBatchUnrollWide; ++k) xv[k] = d.x[static_cast<int64_t>(sv[k]) * B + bl];
-#pragma unroll
-      for (int k = 0; k < kBatchUnrollWide; ++k)
-        if (live[k]) s = Mono<M>::op(s, map_term(d.map, wv[k], xv[k]));
+      for (; j < n; ++j) s = Mono<M>::op(s, term[par][j][smp]);
     }
-    for (; e < e1; ++e) {
-      if (d.dead && d.dead[e]) continue;
-      s = Mono<M>::op(s, map_term(d.map, d.weight[e], d.x[static_cast<int64_t>(d.src[e]) * B + bl]));
-    }
-    if (b < B) finish_batch<M>(d.acc, d.apply, fin, static_cast<int64_t>(u) * B + b, s);
+    // (the other buffer takes the next window: its last reader passed the
+    // barrier above)
   }
-}
-
-// The same forward with one wave per row and four samples per lane (16-byte
-// loads of the gathered rows; B a multiple of 4): each sample's fold is the
-// row's positions in order, as above.
-template <int M>
-__global__ __launch_bounds__(64) void k_forward_batch4(plx_forward_desc d, int32_t B) {
-  const int r = blockIdx.x;
-  const int u = d.row_unit[r];
-  const int e0 = d.row_ptr[r], e1 = d.row_ptr[r + 1];
-  const bool fin = finalizes(d.fin, u);
-  const float ident = Mono<M>::id();
-  for (int b0 = 0; b0 < B; b0 += 256) {
-    const int b = b0 + 4 * static_cast<int>(threadIdx.x);
-    const int bl = b < B ? b : B - 4;  // every lane's loads stay in its row
-    float s[4] = {ident, ident, ident, ident};
-    int e = e0;
-    for (; e + kBatchUnroll <= e1; e += kBatchUnroll) {
-      int sv[kBatchUnroll];
-      float wv[kBatchUnroll];
-      bool live[kBatchUnroll];
-      float4 xv[kBatchUnroll];
-#pragma unroll
-      for (int k = 0; k < kBatchUnroll; ++k) {
-        sv[k] = d.src[e + k];
-        wv[k] = d.weight[e + k];
-        live[k] = d.dead ? d.dead[e + k] == 0 : true;
-      }
-#pragma unroll
-      for (int k = 0; k < kBatchUnroll; ++k)
-        xv[k] = *reinterpret_cast<const float4*>(d.x + static_cast<int64_t>(sv[k]) * B + bl);
-#pragma unroll
-      for (int k = 0; k < kBatchUnroll; ++k) {
-        if (!live[k]) continue;
-        s[0] = Mono<M>::op(s[0], map_term(d.map, wv[k], xv[k].x));
-        s[1] = Mono<M>::op(s[1], map_term(d.map, wv[k], xv[k].y));
-        s[2] = Mono<M>::op(s[2], map_term(d.map, wv[k], xv[k].z));
-        s[3] = Mono<M>::op(s[3], map_term(d.map, wv[k], xv[k].w));
-      }
-    }
-    for (; e < e1; ++e) {
-      if (d.dead && d.dead[e]) continue;
-      const float w = d.weight[e];
-      const float4 x = *reinterpret_cast<const float4*>(d.x + static_cast<int64_t>(d.src[e]) * B + bl);
-      s[0] = Mono<M>::op(s[0], map_term(d.map, w, x.x));
-      s[1] = Mono<M>::op(s[1], map_term(d.map, w, x.y));
-      s[2] = Mono<M>::op(s[2], map_term(d.map, w, x.z));
-      s[3] = Mono<M>::op(s[3], map_term(d.map, w, x.w));
-    }
-    if (b < B)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) finish_batch<M>(d.acc, d.apply, fin, static_cast<int64_t>(u) * B + b + k, s[k]);
-  }
-}
-
-template <int M>
-__global__ __launch_bounds__(kBatchBlock) void k_backward_batch(plx_bwd_batch_desc d) {
-  const int r = blockIdx.x;
-  const int B = d.batch;
-  const int u = d.row_unit[r];
-  const int j0 = d.row_ptr[r], j1 = d.row_ptr[r + 1];
-  const bool fin = finalizes(d.fin, u);
-  const float ident = Mono<M>::id();
-  for (int b0 = 0; b0 < B; b0 += blockDim.x) {
-    const int b = b0 + static_cast<int>(threadIdx.x);
-    const int bl = b < B ? b : B - 1;
-    float s = ident;
-    int j = j0;
-    for (; j + kBatchUnrollWide <= j1; j += kBatchUnrollWide) {
-      int tv[kBatchUnrollWide];
-      float wv[kBatchUnrollWide], gv[kBatchUnrollWide];
-      bool live[kBatchUnrollWide];
-#pragma unroll
-      for (int k = 0; k < kBatchUnrollWide; ++k) {
-        tv[k] = d.dst[j + k];
-        wv[k] = d.weight[j + k];
-        live[k] = d.live ? d.live[j + k] != 0 : true;
-      }
-#pragma unroll
-      for (int k = 0; k < kBatchUnrollWide; ++k) gv[k] = d.g[static_cast<int64_t>(tv[k]) * B + bl];
-#pragma unroll
-      for (int k = 0; k < kBatchUnrollWide; ++k)
-        if (live[k]) s = Mono<M>::op(s, map_term(d.map, wv[k], gv[k]));
-    }
-    for (; j < j1; ++j) {
-      if (d.live && !d.live[j]) continue;
-      s = Mono<M>::op(s, map_term(d.map, d.weight[j], d.g[static_cast<int64_t>(d.dst[j]) * B + bl]));
-    }
-    if (b < B) finish_batch<M>(d.acc, d.apply, fin, static_cast<int64_t>(u) * B + b, s);
-  }
-}
-
-// The same backward with one wave per row and four samples per lane
-// (16-byte loads of the gathered g rows; B a multiple of 4).
-template <int M>
-__global__ __launch_bounds__(64) void k_backward_batch4(plx_bwd_batch_desc d) {
-  const int r = blockIdx.x;
-  const int B = d.batch;
-  const int u = d.row_unit[r];
-  const int j0 = d.row_ptr[r], j1 = d.row_ptr[r + 1];
-  const bool fin = finalizes(d.fin, u);
-  const float ident = Mono<M>::id();
-  for (int b0 = 0; b0 < B; b0 += 256) {
-    const int b = b0 + 4 * static_cast<int>(threadIdx.x);
-    const int bl = b < B ? b : B - 4;
-    float s[4] = {ident, ident, ident, ident};
-    int j = j0;
-    for (; j + kBatchUnroll <= j1; j += kBatchUnroll) {
-      int tv[kBatchUnroll];
-      float wv[kBatchUnroll];
-      bool live[kBatchUnroll];
-      float4 gv[kBatchUnroll];
-#pragma unroll
-      for (int k = 0; k < kBatchUnroll; ++k) {
-        tv[k] = d.dst[j + k];
-        wv[k] = d.weight[j + k];
-        live[k] = d.live ? d.live[j + k] != 0 : true;
-      }
-#pragma unroll
-      for (int k = 0; k < kBatchUnroll; ++k)
-        gv[k] = *reinterpret_cast<const float4*>(d.g + static_cast<int64_t>(tv[k]) * B + bl);
-#pragma unroll
-      for (int k = 0; k < kBatchUnroll; ++k) {
-        if (!live[k]) continue;
-        s[0] = Mono<M>::op(s[0], map_term(d.map, wv[k], gv[k].x));
-        s[1] = Mono<M>::op(s[1], map_term(d.map, wv[k], gv[k].y));
-        s[2] = Mono<M>::op(s[2], map_term(d.map, wv[k], gv[k].z));
-        s[3] = Mono<M>::op(s[3], map_term(d.map, wv[k], gv[k].w));
-      }
-    }
-    for (; j < j1; ++j) {
-      if (d.live && !d.live[j]) continue;
-      const float w = d.weight[j];
-      const float4 g = *reinterpret_cast<const float4*>(d.g + static_cast<int64_t>(d.dst[j]) * B + bl);
-      s[0] = Mono<M>::op(s[0], map_term(d.map, w, g.x));
-      s[1] = Mono<M>::op(s[1], map_term(d.map, w, g.y));
-      s[2] = Mono<M>::op(s[2], map_term(d.map, w, g.z));
-      s[3] = Mono<M>::op(s[3], map_term(d.map, w, g.w));
-    }
-    if (b < B)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) finish_batch<M>(d.acc, d.apply, fin, static_cast<int64_t>(u) * B + b + k, s[k]);
-  }
+  if (sub == 0 && b < B) finish_batch<M>(d.acc, d.apply, finalizes(d.fin, u), static_cast<int64_t>(u) * B + b, s);
 }
 
 // Streaming backward over slot-ordered lists: lane = row (source unit),
@@ -1614,6 +1626,36 @@ int dispatch_rule(const plx_tile_desc& d, size_t lds, hipStream_t s) {
   return PLX_OK;
 }
 
+// A batched level's launch: a wave per row from 256 rows on (a row for every
+// CU), with 16-byte loads where the unit rows are aligned for them and the
+// samples fill at least half of a wave's lanes; fewer rows take the sample
+// groups.
+template <int M, class D>
+int launch_batch_m(const D& d, int32_t batch, hipStream_t s) {
+  const unsigned rows = static_cast<unsigned>(d.nrows);
+  if (d.nrows >= 256) {
+    if (batch % 4 == 0 && batch >= 128)
+      k_batch_rows<M, D, 4><<<dim3(rows, static_cast<unsigned>((batch + 255) / 256)), 64, 0, s>>>(d, batch);
+    else
+      k_batch_rows<M, D, 1><<<dim3(rows, static_cast<unsigned>((batch + 63) / 64)), 64, 0, s>>>(d, batch);
+  } else {
+    const dim3 grid(rows, static_cast<unsigned>((batch + kGroup - 1) / kGroup));
+    k_batch_groups<M, D><<<grid, kBatchBlock, 0, s>>>(d, batch);
+  }
+  return PLX_OK;
+}
+template <class D>
+int launch_batch(const D& d, int32_t batch, hipStream_t s, const char* who) {
+  switch (d.monoid) {
+    case PLX_MONOID_SUM: launch_batch_m<PLX_MONOID_SUM>(d, batch, s); break;
+    case PLX_MONOID_PROD: launch_batch_m<PLX_MONOID_PROD>(d, batch, s); break;
+    case PLX_MONOID_MAX: launch_batch_m<PLX_MONOID_MAX>(d, batch, s); break;
+    case PLX_MONOID_MIN: launch_batch_m<PLX_MONOID_MIN>(d, batch, s); break;
+    default: return fail(PLX_ERR_UNSUPPORTED, (std::string(who) + ": unknown monoid").c_str());
+  }
+  return check_launch(who);
+}
+
 }  // namespace
 
 int plx_detail::cu_count() {
@@ -1914,29 +1956,7 @@ int plx_forward_batch(const plx_forward_desc* d, int32_t batch, void* stream) {
   if (!d->fin.level || !d->fin.is_input)
     return fail(PLX_ERR_INVALID, "plx_forward_batch: fin.level and fin.is_input are required");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const unsigned block = batch >= kBatchBlock ? kBatchBlock : static_cast<unsigned>((batch + 63) / 64 * 64);
-  const unsigned grid = static_cast<unsigned>(d->nrows);
-  if (batch % 4 == 0 && batch >= 128 && d->nrows >= 256) {
-    // 16-byte row loads: x rows are 16-byte aligned when B is a multiple of 4.
-    // (A level of few rows keeps a 256-lane workgroup per row: with one wave
-    // per row it would leave the GPU idle.)
-    switch (d->monoid) {
-      case PLX_MONOID_SUM: k_forward_batch4<PLX_MONOID_SUM><<<grid, 64, 0, s>>>(*d, batch); break;
-      case PLX_MONOID_PROD: k_forward_batch4<PLX_MONOID_PROD><<<grid, 64, 0, s>>>(*d, batch); break;
-      case PLX_MONOID_MAX: k_forward_batch4<PLX_MONOID_MAX><<<grid, 64, 0, s>>>(*d, batch); break;
-      case PLX_MONOID_MIN: k_forward_batch4<PLX_MONOID_MIN><<<grid, 64, 0, s>>>(*d, batch); break;
-      default: return fail(PLX_ERR_UNSUPPORTED, "plx_forward_batch: unknown monoid");
-    }
-    return check_launch("plx_forward_batch");
-  }
-  switch (d->monoid) {
-    case PLX_MONOID_SUM: k_forward_batch<PLX_MONOID_SUM><<<grid, block, 0, s>>>(*d, batch); break;
-    case PLX_MONOID_PROD: k_forward_batch<PLX_MONOID_PROD><<<grid, block, 0, s>>>(*d, batch); break;
-    case PLX_MONOID_MAX: k_forward_batch<PLX_MONOID_MAX><<<grid, block, 0, s>>>(*d, batch); break;
-    case PLX_MONOID_MIN: k_forward_batch<PLX_MONOID_MIN><<<grid, block, 0, s>>>(*d, batch); break;
-    default: return fail(PLX_ERR_UNSUPPORTED, "plx_forward_batch: unknown monoid");
-  }
-  return check_launch("plx_forward_batch");
+  return launch_batch(*d, batch, s, "plx_forward_batch");
 }
 
 int plx_backward_batch(const plx_bwd_batch_desc* d, void* stream) {
@@ -1950,29 +1970,7 @@ int plx_backward_batch(const plx_bwd_batch_desc* d, void* stream) {
   if (!d->fin.level || !d->fin.is_input)
     return fail(PLX_ERR_INVALID, "plx_backward_batch: fin.level and fin.is_input are required");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int batch = d->batch;
-  const unsigned block = batch >= kBatchBlock ? kBatchBlock : static_cast<unsigned>((batch + 63) / 64 * 64);
-  const unsigned grid = static_cast<unsigned>(d->nrows);
-  if (batch % 4 == 0 && batch >= 128 && d->nrows >= 256) {
-    // 16-byte row loads: g rows are 16-byte aligned when B is a multiple of 4
-    // (few rows: the 256-lane form, as for the forward).
-    switch (d->monoid) {
-      case PLX_MONOID_SUM: k_backward_batch4<PLX_MONOID_SUM><<<grid, 64, 0, s>>>(*d); break;
-      case PLX_MONOID_PROD: k_backward_batch4<PLX_MONOID_PROD><<<grid, 64, 0, s>>>(*d); break;
-      case PLX_MONOID_MAX: k_backward_batch4<PLX_MONOID_MAX><<<grid, 64, 0, s>>>(*d); break;
-      case PLX_MONOID_MIN: k_backward_batch4<PLX_MONOID_MIN><<<grid, 64, 0, s>>>(*d); break;
-      default: return fail(PLX_ERR_UNSUPPORTED, "plx_backward_batch: unknown monoid");
-    }
-    return check_launch("plx_backward_batch");
-  }
-  switch (d->monoid) {
-    case PLX_MONOID_SUM: k_backward_batch<PLX_MONOID_SUM><<<grid, block, 0, s>>>(*d); break;
-    case PLX_MONOID_PROD: k_backward_batch<PLX_MONOID_PROD><<<grid, block, 0, s>>>(*d); break;
-    case PLX_MONOID_MAX: k_backward_batch<PLX_MONOID_MAX><<<grid, block, 0, s>>>(*d); break;
-    case PLX_MONOID_MIN: k_backward_batch<PLX_MONOID_MIN><<<grid, block, 0, s>>>(*d); break;
-    default: return fail(PLX_ERR_UNSUPPORTED, "plx_backward_batch: unknown monoid");
-  }
-  return check_launch("plx_backward_batch");
+  return launch_batch(*d, d->batch, s, "plx_backward_batch");
 }
 
 int plx_backward_lists(const plx_bwd_batch_desc* d, void* stream) {
