@@ -1140,7 +1140,68 @@ constexpr int kTileStride = kTileChunk + 4;  // 16-byte aligned rows, offset by 
 constexpr int kTileEdgesPer = 4;
 constexpr int kTileEdges = kTileEdgesPer * kBatchBlock;
 
-template <int RULE, bool UNI_T>
+// What bounds the update is the LDS (8 bytes per edge and sample, random source
+// rows) and, close behind, the instructions per edge and sample, so a lane's
+// edges go two at a time through one loop, unrolled by two steps (no copies of
+// the rows read ahead), and the rows are staged by 16-byte loads: 1.7M edges,
+// 256 samples, 159 -> 136 us; four edges at once, fully unrolled, 185 (224
+// registers: two waves per SIMD).
+//
+// A chunk of cn samples added to the running sums of E of a lane's edges
+// (first: the batch's first chunk, whose sum starts from sample 0's term, not
+// from +0.0). An edge's sum is a chain of adds in sample order, so the lane's
+// edges run side by side, four samples a step, and the next step's rows are
+// read before this step's are added. (A lane without an E-th edge sums row 0
+// for nothing.)
+template <int E>
+__device__ __forceinline__ void tile_sums(const float* gs, const float* as, const int* ld, const int* ls,
+                                          float* total, bool first, int cn) {
+  const float* g[E];
+  const float* a[E];
+  float4 x[E], y[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    g[i] = gs + ld[i] * kTileStride;
+    a[i] = as + ls[i] * kTileStride;
+    x[i] = *reinterpret_cast<const float4*>(g[i]);
+    y[i] = *reinterpret_cast<const float4*>(a[i]);
+  }
+#pragma unroll 2
+  for (int c = 0; c < cn; c += 4) {
+    float4 nx[E], ny[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) {  // (a row's padding is read past its last samples)
+      nx[i] = *reinterpret_cast<const float4*>(g[i] + c + 4 - (c + 4 == kTileChunk ? 4 : 0));
+      ny[i] = *reinterpret_cast<const float4*>(a[i] + c + 4 - (c + 4 == kTileChunk ? 4 : 0));
+    }
+    if (c + 4 <= cn) {
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        const float t = x[i].x * y[i].x;
+        float s = first && c == 0 ? t : total[i] + t;
+        s = s + x[i].y * y[i].y;
+        s = s + x[i].z * y[i].z;
+        total[i] = s + x[i].w * y[i].w;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        const float t = x[i].x * y[i].x;
+        float s = first && c == 0 ? t : total[i] + t;
+        if (c + 1 < cn) s = s + x[i].y * y[i].y;
+        if (c + 2 < cn) s = s + x[i].z * y[i].z;
+        total[i] = s;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      x[i] = nx[i];
+      y[i] = ny[i];
+    }
+  }
+}
+
+template <int RULE, bool UNI_T, int SV>
 __global__ __launch_bounds__(kBatchBlock) void k_update_batch_tiles(plx_update_desc d, plx_batch_tiles t,
                                                                     int32_t B) {
   __shared__ __align__(16) float gs[kTileRows * kTileStride];
@@ -1168,20 +1229,28 @@ __global__ __launch_bounds__(kBatchBlock) void k_update_batch_tiles(plx_update_d
       use[i] = d.dead ? d.dead[pe[i]] == 0 : pe[i] < d.live_end;
     }
   }
+  // Edges a lane: of its wave's lanes, the first holds most.
+  const int first = j0 + (__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x)) & ~63);
+  const int nslot = first < j1 ? (j1 - first + kBatchBlock - 1) / kBatchBlock : 0;
   // Rows [base, base + 64) x samples [c0, c0 + 64) of both fields (rows
   // past the last unit and samples past B are not read) go to registers, every
   // load issued before any is used; the next chunk's loads are in flight while
   // this chunk is summed from LDS.
-  constexpr int kStage = kTileRows * kTileChunk / kBatchBlock;
-  float vg[kStage], va[kStage];
+  constexpr int kWide = kTileChunk / SV;  // loads per row
+  constexpr int kStage = kTileRows * kWide / kBatchBlock;
+  constexpr int kRowStep = kBatchBlock / kWide;  // rows between a thread's loads
+  const int sr = static_cast<int>(threadIdx.x) / kWide, sc = static_cast<int>(threadIdx.x) % kWide * SV;
+  BatchLane<SV> vg[kStage], va[kStage];
   auto stage_load = [&](int c0) {
+    const float* pg = d.gfield + static_cast<int64_t>(dbase + sr) * B + c0 + sc;
+    const float* pa = d.act + static_cast<int64_t>(sbase + sr) * B + c0 + sc;
+    const bool inc = c0 + sc < B;
 #pragma unroll
     for (int i = 0; i < kStage; ++i) {
-      const int q = static_cast<int>(threadIdx.x) + i * kBatchBlock;
-      const int r = q / kTileChunk, c = q % kTileChunk;
-      const bool inc = c0 + c < B;
-      vg[i] = inc && dbase + r < t.num_units ? d.gfield[static_cast<int64_t>(dbase + r) * B + c0 + c] : 0.0f;
-      va[i] = inc && sbase + r < t.num_units ? d.act[static_cast<int64_t>(sbase + r) * B + c0 + c] : 0.0f;
+      const int64_t o = static_cast<int64_t>(i * kRowStep) * B;
+      vg[i] = va[i] = BatchLane<SV>{};
+      if (inc && dbase + sr + i * kRowStep < t.num_units) vg[i] = load_batch<SV>(pg + o);
+      if (inc && sbase + sr + i * kRowStep < t.num_units) va[i] = load_batch<SV>(pa + o);
     }
   };
   stage_load(0);
@@ -1189,43 +1258,24 @@ __global__ __launch_bounds__(kBatchBlock) void k_update_batch_tiles(plx_update_d
     const int cn = min(kTileChunk, B - c0);
 #pragma unroll
     for (int i = 0; i < kStage; ++i) {
-      const int q = static_cast<int>(threadIdx.x) + i * kBatchBlock;
-      const int r = q / kTileChunk, c = q % kTileChunk;
-      gs[r * kTileStride + c] = vg[i];
-      as[r * kTileStride + c] = va[i];
+      float* g = gs + (sr + i * kRowStep) * kTileStride + sc;
+      float* a = as + (sr + i * kRowStep) * kTileStride + sc;
+      if constexpr (SV == 4) {
+        *reinterpret_cast<float4*>(g) = make_float4(vg[i].v[0], vg[i].v[1], vg[i].v[2], vg[i].v[3]);
+        *reinterpret_cast<float4*>(a) = make_float4(va[i].v[0], va[i].v[1], va[i].v[2], va[i].v[3]);
+      } else {
+        *g = vg[i].v[0];
+        *a = va[i].v[0];
+      }
     }
     __syncthreads();
     if (c0 + kTileChunk < B) stage_load(c0 + kTileChunk);
 #pragma unroll
-    for (int i = 0; i < kTileEdgesPer; ++i) {
-      if (!use[i]) continue;
-      const float* g = gs + ld[i] * kTileStride;
-      const float* a = as + ls[i] * kTileStride;
-      float s = total[i];
-      int c = 0;
-      if (c0 == 0) {
-        s = g[0] * a[0];  // the sum starts from sample 0's term, not from +0.0
-        c = 1;
-      }
-      // Up to the next multiple of 4 one sample at a time, then eight
-      // samples per step from 16-byte LDS reads.
-      for (; c < cn && (c & 3); ++c) s = s + g[c] * a[c];
-      for (; c + 8 <= cn; c += 8) {
-        const float4 x0 = *reinterpret_cast<const float4*>(g + c);
-        const float4 x1 = *reinterpret_cast<const float4*>(g + c + 4);
-        const float4 y0 = *reinterpret_cast<const float4*>(a + c);
-        const float4 y1 = *reinterpret_cast<const float4*>(a + c + 4);
-        s = s + x0.x * y0.x;
-        s = s + x0.y * y0.y;
-        s = s + x0.z * y0.z;
-        s = s + x0.w * y0.w;
-        s = s + x1.x * y1.x;
-        s = s + x1.y * y1.y;
-        s = s + x1.z * y1.z;
-        s = s + x1.w * y1.w;
-      }
-      for (; c < cn; ++c) s = s + g[c] * a[c];
-      total[i] = s;
+    for (int i = 0; i < kTileEdgesPer; i += 2) {  // (nslot is uniform over the wave)
+      if (nslot > i + 1)
+        tile_sums<2>(gs, as, ld + i, ls + i, total + i, c0 == 0, cn);
+      else if (nslot > i)
+        tile_sums<1>(gs, as, ld + i, ls + i, total + i, c0 == 0, cn);
     }
     __syncthreads();
   }
@@ -1656,6 +1706,30 @@ int launch_batch(const D& d, int32_t batch, hipStream_t s, const char* who) {
   return check_launch(who);
 }
 
+template <int SV>
+int launch_batch_tiles(const plx_update_desc& d, const plx_batch_tiles& t, int32_t batch, hipStream_t s) {
+  const unsigned grid = static_cast<unsigned>(t.ntiles);
+  switch (d.rule) {
+    case PLX_RULE_SGD:
+      k_update_batch_tiles<PLX_RULE_SGD, false, SV><<<grid, kBatchBlock, 0, s>>>(d, t, batch);
+      break;
+    case PLX_RULE_MOMENTUM:
+      k_update_batch_tiles<PLX_RULE_MOMENTUM, false, SV><<<grid, kBatchBlock, 0, s>>>(d, t, batch);
+      break;
+    case PLX_RULE_ADAM:
+      if (d.step_mode == 1)
+        k_update_batch_tiles<PLX_RULE_ADAM, true, SV><<<grid, kBatchBlock, 0, s>>>(d, t, batch);
+      else
+        k_update_batch_tiles<PLX_RULE_ADAM, false, SV><<<grid, kBatchBlock, 0, s>>>(d, t, batch);
+      break;
+    case PLX_RULE_RMSPROP:
+      k_update_batch_tiles<PLX_RULE_RMSPROP, false, SV><<<grid, kBatchBlock, 0, s>>>(d, t, batch);
+      break;
+    default: return fail(PLX_ERR_UNSUPPORTED, "plx_update_batch_tiles: unknown rule");
+  }
+  return PLX_OK;
+}
+
 }  // namespace
 
 int plx_detail::cu_count() {
@@ -2062,23 +2136,9 @@ int plx_update_batch_tiles(const plx_update_desc* d, const plx_batch_tiles* t, i
   if (d->rule == PLX_RULE_ADAM && (!d->s0 || !d->s1 || (d->step_mode == 0 && !d->s2)))
     return fail(PLX_ERR_INVALID, "plx_update_batch_tiles: Adam state columns missing");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const unsigned grid = static_cast<unsigned>(t->ntiles);
-  switch (d->rule) {
-    case PLX_RULE_SGD: k_update_batch_tiles<PLX_RULE_SGD, false><<<grid, kBatchBlock, 0, s>>>(*d, *t, batch); break;
-    case PLX_RULE_MOMENTUM:
-      k_update_batch_tiles<PLX_RULE_MOMENTUM, false><<<grid, kBatchBlock, 0, s>>>(*d, *t, batch);
-      break;
-    case PLX_RULE_ADAM:
-      if (d->step_mode == 1)
-        k_update_batch_tiles<PLX_RULE_ADAM, true><<<grid, kBatchBlock, 0, s>>>(*d, *t, batch);
-      else
-        k_update_batch_tiles<PLX_RULE_ADAM, false><<<grid, kBatchBlock, 0, s>>>(*d, *t, batch);
-      break;
-    case PLX_RULE_RMSPROP:
-      k_update_batch_tiles<PLX_RULE_RMSPROP, false><<<grid, kBatchBlock, 0, s>>>(*d, *t, batch);
-      break;
-    default: return fail(PLX_ERR_UNSUPPORTED, "plx_update_batch_tiles: unknown rule");
-  }
+  // (16-byte staging where the unit rows are aligned for it)
+  const int rc = batch % 4 == 0 ? launch_batch_tiles<4>(*d, *t, batch, s) : launch_batch_tiles<1>(*d, *t, batch, s);
+  if (rc) return rc;
   return check_launch("plx_update_batch_tiles");
 }
 
