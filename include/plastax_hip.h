@@ -414,6 +414,20 @@ PLX_EXPORT int plx_loss_elementwise_batch(int32_t n_out, const int32_t* output_i
 /* StepResult.loss of a batched step (step.py:466): (0 + l_0 + ... + l_{B-1}) / B. */
 PLX_EXPORT int plx_batch_mean(int32_t batch, const float* losses, float* out, void* stream);
 
+/* A batched step's column copies, up to PLX_MAX_BATCH_COLS columns a launch
+ * (src, dst, modes: host arrays). plx_spread_cols: dst[j][u * batch + b] =
+ * src[j][u] (4-byte values): every sample starts from the shared state
+ * (step.py:421-424). plx_scatter_batch: the inputs, dst[ids[k] * batch + b] =
+ * values[b * n + k] (step.py:598 per sample). plx_reduce_cols: plx_reduce_batch
+ * of float32 columns. */
+#define PLX_MAX_BATCH_COLS 8
+PLX_EXPORT int plx_spread_cols(int64_t n, int32_t batch, int32_t ncols, const void* const* src, void* const* dst,
+                               void* stream);
+PLX_EXPORT int plx_scatter_batch(int32_t n, int32_t batch, const int32_t* ids, const float* values, float* dst,
+                                 void* stream);
+PLX_EXPORT int plx_reduce_cols(int64_t n, int32_t batch, int32_t ncols, const int32_t* modes,
+                               const void* const* src, void* const* dst, void* stream);
+
 /* reduce_batch_units (phases.py:298-332) for one column: dst[u] from
  * src[u * B .. u * B + B): PLX_REDUCE_MEAN (float32: x_0 + x_1 + ... in
  * sample order, then / B), PLX_REDUCE_SUM (the same sum; int32 wraps),

@@ -27,6 +27,7 @@ PLX_MAX_OUTS = 4
 PLX_MAX_TBL = 8192
 PLX_SOFTMAX_ONE = 4096
 PLX_MAX_SLOT_COLS = 8
+PLX_MAX_BATCH_COLS = 8
 PLX_MAX_SINSTR = 160
 PLX_MAX_SCONST = 32
 PLX_MAX_SFIELDS = 8
@@ -546,6 +547,9 @@ _SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "plx_gen_fold": (c_i32, [ctypes.POINTER(plx_gen_fold_desc), c_vp]),
     "plx_copy_to_slots": (c_i32, [c_i64, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i32, c_vp]),
     "plx_merge_index": (c_i32, [ctypes.POINTER(plx_merge_desc), c_vp]),
+    "plx_spread_cols": (c_i32, [c_i64, c_i32, c_i32, c_vp, c_vp, c_vp]),
+    "plx_scatter_batch": (c_i32, [c_i32, c_i32, c_vp, c_vp, c_vp, c_vp]),
+    "plx_reduce_cols": (c_i32, [c_i64, c_i32, c_i32, c_vp, c_vp, c_vp, c_vp]),
     "plx_write_slots": (c_i32, [c_i64, c_vp, c_vp, c_i64, c_i32, c_vp, c_vp, c_vp, ctypes.c_uint32, c_vp, c_i64, c_vp]),
     "plx_fill_live": (c_i32, [c_i64, c_vp, c_f32, c_vp, c_vp]),
     "plx_merge_gather": (c_i32, [ctypes.POINTER(plx_merge_gather_desc), c_vp]),

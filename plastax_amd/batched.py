@@ -72,6 +72,23 @@ def batch_sources(arena: Arena, b: int) -> BatchSources:
     return cache[b]
 
 
+def top_sources(arena: Arena) -> BatchSources:
+    """The deepest level's rows, whose lists are empty (kept with the arena)."""
+    if "_top_sources" not in arena.__dict__:
+        top = arena.top
+        zeros = torch.zeros(top.nrows + 1, dtype=torch.int32, device=arena.device)
+        arena._top_sources = BatchSources(top.nrows, top.rows, zeros, zeros, zeros)
+    return arena._top_sources
+
+
+def _pointers(tensors: list[torch.Tensor]) -> Any:
+    return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+
+
+def _chunks(names: list[str], size: int) -> list[list[str]]:
+    return [names[k : k + size] for k in range(0, len(names), size)]
+
+
 def batch_sources_host(arena: Arena, b: int) -> BatchSources:
     """batch_sources built on the host with numpy (the restatement the
     device build is tested against)."""
@@ -156,7 +173,7 @@ class BatchedStepFn(StepFn):
                 raise ValueError(f"{net.__name__}.{err}") from None
         return out
 
-    def _batched_columns(self, units: dict[str, torch.Tensor], g: Any) -> dict[str, torch.Tensor]:
+    def _batched_columns(self, units: dict[str, torch.Tensor], g: Any, stream: int) -> dict[str, torch.Tensor]:
         """[num_units, B] copies of every column a per-sample phase reads or
         writes (each sample starts from the shared state: step.py:421-424)."""
         plan = self.plan
@@ -188,7 +205,19 @@ class BatchedStepFn(StepFn):
             names.update(n for n in p.fields)
             names.update(n for n in p.out_fields if n is not None)
         B = self.batch
-        return {n: units[n].unsqueeze(1).expand(-1, B).contiguous() for n in sorted(names)}
+        out = {}
+        words = []
+        for n in sorted(names):
+            if units[n].element_size() == 4:
+                words.append(n)
+                out[n] = torch.empty((units[n].numel(), B), dtype=units[n].dtype, device=units[n].device)
+            else:
+                out[n] = units[n].unsqueeze(1).expand(-1, B).contiguous()
+        for part in _chunks(words, _lib.PLX_MAX_BATCH_COLS):
+            src, dst = _pointers([units[n] for n in part]), _pointers([out[n] for n in part])
+            _lib.call("plx_spread_cols", int(units[part[0]].numel()), B, len(part), ctypes.addressof(src),
+                      ctypes.addressof(dst), stream)
+        return out
 
     def __call__(self, state: NetworkState, inputs: StepInputs) -> StepResult:
         from plastax_amd import grow
@@ -226,9 +255,11 @@ class BatchedStepFn(StepFn):
         units = state._physical_units(arena)
         n_units = self.static.num_units
         g = state.globals_
-        ub = self._batched_columns(units, g)
+        ub = self._batched_columns(units, g, stream)
         if n_in:
-            ub[ACTIVATION.name][consts["input_ids"].long()] = x.t()
+            x = x.contiguous()
+            _lib.call("plx_scatter_batch", n_in, B, consts["input_ids"].data_ptr(), x.data_ptr(),
+                      ub[ACTIVATION.name].data_ptr(), stream)
         fin = dict(
             level=units["level"].data_ptr(),
             is_input=consts["is_input"].data_ptr(),
@@ -276,7 +307,7 @@ class BatchedStepFn(StepFn):
             self._launch("forward", lib.plx_forward_batch, d, B, stream)
 
         # Loss, per sample, then the batch mean (step.py:448-451, :466).
-        loss = torch.zeros((), dtype=torch.float32, device=dev)
+        loss = (torch.zeros if plan.loss is None else torch.empty)((), dtype=torch.float32, device=dev)
         if plan.loss is not None:
             if t is None:
                 raise ValueError("step: this net has a loss, so StepInputs.targets is required")
@@ -321,7 +352,6 @@ class BatchedStepFn(StepFn):
             if arena.bwd_carry:
                 bacc = torch.full((n_units, B), bp.identity, dtype=torch.float32, device=dev)
             bprog = program_struct(bp.program, ub, g)
-            empty = torch.zeros(1, dtype=torch.int32, device=dev)
 
             def run(rows: torch.Tensor, nrows: int, ptr: torch.Tensor, lists: Any, level: int) -> None:
                 d = _lib.plx_bwd_batch_desc()
@@ -348,9 +378,8 @@ class BatchedStepFn(StepFn):
             nb = arena.num_buckets
             top = arena.top
             if top.nrows:
-                zeros = torch.zeros(top.nrows + 1, dtype=torch.int32, device=dev)
-                none = BatchSources(0, empty, empty, empty, empty)
-                run(top.rows, top.nrows, zeros, none, nb)
+                none = top_sources(arena)
+                run(none.rows, none.nrows, none.ptr, none, nb)
             for b in range(nb - 1, 0, -1):
                 lists = batch_sources(arena, b)
                 run(lists.rows, lists.nrows, lists.ptr, lists, b)
@@ -374,9 +403,17 @@ class BatchedStepFn(StepFn):
             state._mark_ahead()
 
         # reduce_batch_units (phases.py:298-332): the written columns only.
+        floats = [name for name in reductions if units[name].dtype == torch.float32]
+        for part in _chunks(floats, _lib.PLX_MAX_BATCH_COLS):
+            src, dst = _pointers([ub[name] for name in part]), _pointers([units[name] for name in part])
+            modes = (ctypes.c_int32 * len(part))(*[_REDUCE[reductions[name]] for name in part])
+            _lib.call("plx_reduce_cols", n_units, B, len(part), ctypes.addressof(modes), ctypes.addressof(src),
+                      ctypes.addressof(dst), stream)
         for name, red in reductions.items():
             col = units[name]
-            kind = 0 if col.dtype == torch.float32 else (1 if col.dtype == torch.int32 else 2)
+            if col.dtype == torch.float32:
+                continue
+            kind = 1 if col.dtype == torch.int32 else 2
             _lib.check(
                 lib.plx_reduce_batch(n_units, B, _REDUCE[red], kind, ub[name].data_ptr(), col.data_ptr(), stream),
                 "plx_reduce_batch",
