@@ -446,6 +446,11 @@ PLX_EXPORT int plx_reduce_batch(int64_t n, int32_t batch, int32_t mode, int32_t 
 PLX_EXPORT int plx_scatter_f32(int32_t n, const int32_t* ids, const float* values,
                     float* dst, void* stream);
 
+/* The same into two columns (also may be null): a PIPELINE step's activations
+ * and the column its forward writes, whose input units the forward skips. */
+PLX_EXPORT int plx_scatter_pair_f32(int32_t n, const int32_t* ids, const float* values,
+                         float* dst, float* also, void* stream);
+
 /* Elementwise loss (phases.py:1107-1131 with a policy whose seed and loss
  * term are elementwise in (prediction, target), e.g. MSE): `term` writes out
  * slot 0 (the seed) to seed_field[output_ids[k]]; slot 1 is the loss term.

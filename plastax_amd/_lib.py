@@ -493,6 +493,7 @@ _SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "plx_roof_probe": (c_i32, [c_i32, c_i32, c_vp, c_i64, c_vp, ctypes.POINTER(ctypes.c_double),
                                ctypes.POINTER(ctypes.c_float), c_vp]),
     "plx_update_conn": (c_i32, [ctypes.POINTER(plx_update_desc), c_vp]),
+    "plx_scatter_pair_f32": (c_i32, [c_i32, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "plx_scatter_f32": (c_i32, [c_i32, c_vp, c_vp, c_vp, c_vp]),
     "plx_loss_elementwise": (
         c_i32,

@@ -263,6 +263,13 @@ class StepFn:
         units = state._physical_units(arena)
         n_units = self.static.num_units
 
+        # A PIPELINE forward writes every unit but the inputs, whose new values
+        # the scatter places (units may be pruned: then a copy keeps them).
+        swaps: dict[str, torch.Tensor] = {}
+        if arena.pipeline and plan.forward.generic is None:
+            every = () if "pruned" in units else (ACTIVATION.name,)
+            swaps = self._shadow(units, plan.forward.program.out_fields, every)
+
         # Input scatter (step.py:598).
         n_in = len(self.static.input_ids)
         if n_in:
@@ -271,11 +278,12 @@ class StepFn:
             if x_in.numel() != n_in:
                 raise ValueError(f"step: expected {n_in} inputs, got {x_in.numel()}")
             _lib.check(
-                lib.plx_scatter_f32(
+                lib.plx_scatter_pair_f32(
                     n_in,
                     consts["input_ids"].data_ptr(),
                     x_in.data_ptr(),
                     units[ACTIVATION.name].data_ptr(),
+                    swaps[ACTIVATION.name].data_ptr() if ACTIVATION.name in swaps else None,
                     stream,
                 ),
                 "plx_scatter_f32",
@@ -293,7 +301,6 @@ class StepFn:
             self._forward_generic(arena, units, g, stream)
         else:
             fp = plan.forward
-            swaps = self._shadow(units, fp.program.out_fields) if arena.pipeline else {}
             acc = None
             if arena.fwd_carry:
                 acc = torch.empty(n_units, dtype=torch.float32, device=dev)
@@ -650,10 +657,19 @@ class StepFn:
 
     # -- phases -----------------------------------------------------------------
     @staticmethod
-    def _shadow(units: dict[str, torch.Tensor], out_fields: list[str | None]) -> dict[str, torch.Tensor]:
+    def _shadow(units: dict[str, torch.Tensor], out_fields: list[str | None],
+                every: tuple[str, ...] = ()) -> dict[str, torch.Tensor]:
         """PIPELINE applies write every unit at once against the pre-phase
-        columns (sweep.py:205-228): write into copies, swapped in after."""
-        return {f: units[f].clone() for f in out_fields if f is not None}
+        columns (sweep.py:205-228): write into copies, swapped in after (of
+        the fields in ``every`` each unit is written, so nothing is copied)."""
+        return {f: torch.empty_like(units[f]) if f in every else units[f].clone()
+                for f in out_fields if f is not None}
+
+    def _shadow_backward(self, units: dict[str, torch.Tensor], bp: Any) -> dict[str, torch.Tensor]:
+        """A PIPELINE backward applies every unit, inputs included
+        (sweep.py:442-447), but a pruned one."""
+        fields = bp.program.out_fields
+        return self._shadow(units, fields, () if "pruned" in units else tuple(f for f in fields if f))
 
     @staticmethod
     def _unshadow(units: dict[str, torch.Tensor], swaps: dict[str, torch.Tensor]) -> None:
@@ -797,7 +813,7 @@ class StepFn:
         dev = arena.device
         n = self.static.num_units
         nb = arena.num_buckets
-        swaps = self._shadow(units, bp.program.out_fields) if arena.pipeline else {}
+        swaps = self._shadow_backward(units, bp) if arena.pipeline else {}
         acc = torch.empty(n, dtype=torch.float32, device=dev)
         _lib.call("plx_fill_f32", n, bp.identity, acc.data_ptr(), stream)
         prog = program_struct(bp.program, units, g, out_override=swaps)
@@ -870,7 +886,7 @@ class StepFn:
         if bp is not None:
             dev = arena.device
             n_units = self.static.num_units
-            swaps = self._shadow(units, bp.program.out_fields) if arena.pipeline else {}
+            swaps = self._shadow_backward(units, bp) if arena.pipeline else {}
             acc = None
             if arena.bwd_carry:
                 acc = torch.empty(n_units, dtype=torch.float32, device=dev)
