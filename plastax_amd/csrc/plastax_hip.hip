@@ -831,8 +831,8 @@ __device__ __forceinline__ int batch_pos(const plx_forward_desc&, int e) { retur
 __device__ __forceinline__ int batch_pos(const plx_bwd_batch_desc& d, int e) { return d.pos ? d.pos[e] : e; }
 __device__ __forceinline__ const uint8_t* batch_dead(const plx_forward_desc& d) { return d.dead; }
 __device__ __forceinline__ const uint8_t* batch_dead(const plx_bwd_batch_desc& d) { return d.dead; }
-__device__ __forceinline__ const float* batch_rows(const plx_forward_desc& d) { return d.x; }
-__device__ __forceinline__ const float* batch_rows(const plx_bwd_batch_desc& d) { return d.g; }
+__host__ __device__ __forceinline__ const float* batch_rows(const plx_forward_desc& d) { return d.x; }
+__host__ __device__ __forceinline__ const float* batch_rows(const plx_bwd_batch_desc& d) { return d.g; }
 
 // Levels of many rows: a wave per row and 64 V samples, V samples per lane (V =
 // 4: 16-byte loads, B a multiple of 4). It gathers a B-wide unit row per edge
@@ -1748,6 +1748,9 @@ int dispatch_rule(const plx_tile_desc& d, size_t lds, hipStream_t s) {
   return PLX_OK;
 }
 
+// (16-byte loads take rows that start on 16 bytes)
+bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
 // A batched level's launch: a wave per row from 256 rows on (a row for every
 // CU), with 16-byte loads where the unit rows are aligned for them and the
 // samples fill at least half of a wave's lanes; fewer rows take the sample
@@ -1756,7 +1759,7 @@ template <int M, class D>
 int launch_batch_m(const D& d, int32_t batch, hipStream_t s) {
   const unsigned rows = static_cast<unsigned>(d.nrows);
   if (d.nrows >= 256) {
-    if (batch % 4 == 0 && batch >= 128)
+    if (batch % 4 == 0 && batch >= 128 && aligned16(batch_rows(d)))
       k_batch_rows<M, D, 4><<<dim3(rows, static_cast<unsigned>((batch + 255) / 256)), 64, 0, s>>>(d, batch);
     else
       k_batch_rows<M, D, 1><<<dim3(rows, static_cast<unsigned>((batch + 63) / 64)), 64, 0, s>>>(d, batch);
@@ -2213,7 +2216,8 @@ int plx_update_batch_tiles(const plx_update_desc* d, const plx_batch_tiles* t, i
     return fail(PLX_ERR_INVALID, "plx_update_batch_tiles: Adam state columns missing");
   hipStream_t s = static_cast<hipStream_t>(stream);
   // (16-byte staging where the unit rows are aligned for it)
-  const int rc = batch % 4 == 0 ? launch_batch_tiles<4>(*d, *t, batch, s) : launch_batch_tiles<1>(*d, *t, batch, s);
+  const bool wide = batch % 4 == 0 && aligned16(d->gfield) && aligned16(d->act);
+  const int rc = wide ? launch_batch_tiles<4>(*d, *t, batch, s) : launch_batch_tiles<1>(*d, *t, batch, s);
   if (rc) return rc;
   return check_launch("plx_update_batch_tiles");
 }
@@ -2307,7 +2311,7 @@ int plx_spread_cols(int64_t n, int32_t batch, int32_t ncols, const void* const* 
     if (!src[j] || !dst[j]) return fail(PLX_ERR_INVALID, "plx_spread_cols: null column");
     c.src[j] = static_cast<const uint32_t*>(src[j]);
     c.dst[j] = static_cast<uint32_t*>(dst[j]);
-    quads = quads && reinterpret_cast<uintptr_t>(dst[j]) % 16 == 0;
+    quads = quads && aligned16(dst[j]);
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 grid(grid_for(n * batch / (quads ? 4 : 1), kBatchBlock), static_cast<unsigned>(ncols));
