@@ -18,8 +18,8 @@ reference's examples xmc.py, upgd.py, cbp.py) -- runs here:
 - the apply is traced into a unit program reading the accumulator from
   those columns (``_site.trace_pass_apply``), evaluated for the units the
   bucket finalizes against the pre-apply columns, its writes committed with
-  ``plx_unit_write`` (pruned units skipped), and the finalized units'
-  accumulators reset to the identity.
+  ``plx_unit_write`` (pruned units skipped). A pass finalizes a unit once and
+  makes its own accumulators, so a finalized unit's are not reset.
 
 The finalize sets are the product path's: forward, level b + 1 after bucket
 b (PIPELINE: every non-input unit after one sweep); backward, the deepest
@@ -36,7 +36,7 @@ pass per sample against the shared connections).
 from __future__ import annotations
 
 import ctypes
-from typing import Any
+from typing import Any, NamedTuple
 
 import numpy as np
 import torch
@@ -111,43 +111,46 @@ class GenericPassRunner:
         _lib.check(k.lib.plx_gen_fold(d, k.s), "plx_gen_fold")
 
     def apply(self, k: Any, arena: Any, units: dict, acc: list[torch.Tensor], g: Any,
-              fin: torch.Tensor, batch: int = 1, pruned: torch.Tensor | None = None) -> None:
-        """The apply on the units ``fin`` (physical ids), against the
-        pre-apply columns; their accumulators go back to the identity.
+              fin: Finalized, batch: int = 1, pruned: torch.Tensor | None = None) -> None:
+        """The apply on the units ``fin``, against the pre-apply columns.
         Pruned units (``pruned``, else the ``pruned`` column) keep their
         columns."""
         from plastax_amd.grow import _ptr
         from plastax_amd.units import _unit_cols
 
-        m = int(fin.numel())
-        if m == 0:
+        m = int(fin.units.numel())
+        if m == 0 or not self.names:
             return
         B = int(batch)
         if pruned is None:
             pruned = units.get("pruned")
         ext = dict(units)
         ext.update(dict(zip(self.acc_names, acc)))
-        idx = fin.long()
-        if self.names:
-            n = m * B
-            at, skip = fin, pruned
-            if B > 1:  # sites (unit, sample), written at unit * B + sample
-                at = (idx[:, None] * B + torch.arange(B, device=idx.device)).reshape(-1).to(torch.int32)
-                skip = None if pruned is None else pruned.repeat_interleave(B)
-            outs = [k.mem.i32(n) for _ in self.names]
-            k.site_eval(self.apply_prog, ext, g, n=n, kind=0, per=1, num_units=self.static.num_units, outs=outs,
-                        site_ids=arena.uperm32[idx].contiguous(), ids_physical=arena.uinv32, batch=B)
-            cols = _unit_cols(units, self.specs, self.names)
-            ptrs = (ctypes.c_void_p * len(outs))(*[o.data_ptr() for o in outs])
-            _lib.check(k.lib.plx_unit_write(n, None, at.data_ptr(), _ptr(skip), len(self.names),
-                                            ctypes.addressof(cols), ctypes.addressof(ptrs), k.s), "plx_unit_write")
-        for a, v in zip(acc, self.gp.identities):
-            a.view(-1, B).index_fill_(0, idx, v)
+        n = m * B
+        at, skip = fin.units, pruned
+        if B > 1:  # sites (unit, sample), written at unit * B + sample
+            at = (at.long()[:, None] * B + torch.arange(B, device=at.device)).reshape(-1).to(torch.int32)
+            skip = None if pruned is None else pruned.repeat_interleave(B)
+        outs = [k.mem.i32(n) for _ in self.names]
+        k.site_eval(self.apply_prog, ext, g, n=n, kind=0, per=1, num_units=self.static.num_units, outs=outs,
+                    site_ids=fin.sites, ids_physical=arena.uinv32, batch=B)
+        cols = _unit_cols(units, self.specs, self.names)
+        ptrs = (ctypes.c_void_p * len(outs))(*[o.data_ptr() for o in outs])
+        _lib.check(k.lib.plx_unit_write(n, None, at.data_ptr(), _ptr(skip), len(self.names),
+                                        ctypes.addressof(cols), ctypes.addressof(ptrs), k.s), "plx_unit_write")
 
 
-def finalize_lists(arena: Any, static: Any) -> dict[str, list[torch.Tensor]]:
-    """Per arena: the units each bucket's apply finalizes (physical ids),
-    forward and backward (see the module docstring)."""
+class Finalized(NamedTuple):
+    """Units a bucket's apply finalizes: their ids in the arena's numbering
+    (``units``) and in the caller's (``sites``), kept with the arena."""
+
+    units: torch.Tensor
+    sites: torch.Tensor
+
+
+def finalize_lists(arena: Any, static: Any) -> dict[str, list[Finalized]]:
+    """Per arena: the units each bucket's apply finalizes, forward and
+    backward (see the module docstring)."""
     cache = arena.__dict__.get("_generic_fin")
     if cache is not None:
         return cache
@@ -158,8 +161,9 @@ def finalize_lists(arena: Any, static: Any) -> dict[str, list[torch.Tensor]]:
         is_input[arena.uinv[np.asarray(static.input_ids, dtype=np.int64)]] = True
     nb = arena.num_buckets
 
-    def lst(mask: np.ndarray) -> torch.Tensor:
-        return torch.from_numpy(np.flatnonzero(mask).astype(np.int32)).to(arena.device)
+    def lst(mask: np.ndarray) -> Finalized:
+        ids = torch.from_numpy(np.flatnonzero(mask).astype(np.int32)).to(arena.device)
+        return Finalized(ids, arena.uperm32[ids.long()].contiguous())
 
     if arena.pipeline:
         fwd = [lst(~is_input)]

@@ -519,9 +519,9 @@ class StepFn:
         fin = finalize_lists(arena, self.static)["bwd"]
         n = self.static.num_units
         acc = run.new_acc(n, arena.device)
-        rows = torch.arange(n, dtype=torch.int32, device=arena.device)
         nb = arena.num_buckets
         churn = hasattr(arena, "lists")
+        rows = torch.arange(n, dtype=torch.int32, device=arena.device) if churn else None
         if arena.pipeline:
             if not churn:
                 raise UnsupportedPolicyError("a generic backward on a PIPELINE net runs on the churn layout")
