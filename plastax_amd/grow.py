@@ -253,10 +253,11 @@ class Kernels:
             d.keys[k].kind, d.keys[k].bits = int(kind), int(bits)
             d.keys[k].bound = int(key[4]) if len(key) > 4 else 0
             d.keys[k].a, d.keys[k].b = a.data_ptr(), _ptr(b)
-        kb, ka, va = self.mem.i32(n_max), self.mem.i32(n_max), self.mem.i32(n_max)
-        hist = self.mem.ints_for(n_max)
+        span = -(-n_max // 64) * 64  # (each buffer starts on a line)
+        work = self.mem.i32(3 * span + int(self.lib.plx_scratch_ints(n_max)))
+        at = work.data_ptr()
         d.vals, d.keys_buf, d.keys_alt, d.vals_alt, d.hist = (
-            vals.data_ptr(), kb.data_ptr(), ka.data_ptr(), va.data_ptr(), hist.data_ptr())
+            vals.data_ptr(), at, at + 4 * span, at + 8 * span, at + 12 * span)
         self._begin(tag)
         _lib.check(self.lib.plx_sort(d, self.s), "plx_sort")
         self._end(tag)
