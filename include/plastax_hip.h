@@ -317,13 +317,13 @@ PLX_EXPORT int plx_forward_batch(const plx_forward_desc* d, int32_t batch, void*
 /* Backward of one bucket for B samples (build_csr_backward, phases.py:843-934,
  * and the reference's per-sample scatter order): row r is source unit
  * row_unit[r]; its out-edges are the list entries j in [row_ptr[r],
- * row_ptr[r+1]) in logical slot order, entry j contributing weight[j] *
- * g[dst[j] * B + b] (pre-update weights) where live[j] is nonzero, folded in
- * that order from the identity, combined into acc (null: the identity) and,
- * where the row finalizes, `apply` runs (fields and outs batched) and acc
- * resets. The lists are slot-ordered copies of the arena's columns
- * (plx_gather_edges); a factor the map holds constant (plx_map flags) is
- * not loaded, so its copy need not exist. */
+ * row_ptr[r+1]) in logical slot order, entry j contributing weight[p] *
+ * g[dst[j] * B + b] (pre-update weights; p is pos[j], or j where pos is null)
+ * unless live[j] is zero or dead[p] is not, folded in that order from the
+ * identity, combined into acc (null: the identity) and, where the row
+ * finalizes, `apply` runs (fields and outs batched) and acc resets. With pos,
+ * weight and dead are the arena's columns; without, weight and live are
+ * slot-ordered copies of them (plx_gather_edges). */
 typedef struct plx_bwd_batch_desc {
   int32_t nrows;
   int32_t monoid;
@@ -333,9 +333,9 @@ typedef struct plx_bwd_batch_desc {
   const int32_t* row_ptr;
   const int32_t* dst;    /* [entries] TO_ID */
   const float* weight;   /* [entries] WEIGHT (with pos: [positions]) */
-  const uint8_t* live;   /* [entries] 0: skipped (null: every entry live; plx_backward_lists) */
+  const uint8_t* live;   /* [entries] 0: skipped (null: none is) */
   const int32_t* pos;    /* [entries] the entry's position in weight and dead, or null: the entry itself */
-  const uint8_t* dead;   /* non-zero: skipped (null: none is; plx_backward_batch) */
+  const uint8_t* dead;   /* [positions] non-zero: skipped (null: none is) */
   const float* g;        /* [num_units][B] the map's linear_input field */
   float* acc;            /* [num_units][B] carried accumulator, or null */
   plx_finalize fin;
@@ -347,8 +347,11 @@ PLX_EXPORT int plx_backward_batch(const plx_bwd_batch_desc* d, void* stream);
 
 /* The streaming backward of one bucket over the same slot-ordered lists
  * (batch must be 1): one lane per row, each folding its list in slot order
- * (the reference's per-source scatter order, sweep.py:343-399). Used by the
- * churn layout, which rebuilds on the device after every structural change. */
+ * (the reference's per-source scatter order, sweep.py:343-399). weight and
+ * live are in list order: pos and dead must be null. A factor the map holds
+ * constant (plx_map flags) is not loaded, so its copy need not exist. Used by
+ * the churn layout, which rebuilds on the device after every structural
+ * change. */
 PLX_EXPORT int plx_backward_lists(const plx_bwd_batch_desc* d, void* stream);
 
 /* out_weight[j] = weight[pos[j]] (out_weight optional), out_live[j] =

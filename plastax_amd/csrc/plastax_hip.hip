@@ -824,13 +824,18 @@ __device__ __forceinline__ void finish_batch(float* acc, const plx_program& P, b
 
 // Entries of a batched row, the same for both directions: a forward row's
 // positions (source, weight, tombstone), a backward row's list entries
-// (destination; weight and tombstone of the position they name).
+// (destination, liveness; weight and tombstone of the position they name).
 __device__ __forceinline__ const int32_t* batch_other(const plx_forward_desc& d) { return d.src; }
 __device__ __forceinline__ const int32_t* batch_other(const plx_bwd_batch_desc& d) { return d.dst; }
 __device__ __forceinline__ int batch_pos(const plx_forward_desc&, int e) { return e; }
 __device__ __forceinline__ int batch_pos(const plx_bwd_batch_desc& d, int e) { return d.pos ? d.pos[e] : e; }
-__device__ __forceinline__ const uint8_t* batch_dead(const plx_forward_desc& d) { return d.dead; }
-__device__ __forceinline__ const uint8_t* batch_dead(const plx_bwd_batch_desc& d) { return d.dead; }
+// Whether any entry may be skipped, and whether entry e (at position p) is.
+__device__ __forceinline__ bool batch_skips(const plx_forward_desc& d) { return d.dead; }
+__device__ __forceinline__ bool batch_skips(const plx_bwd_batch_desc& d) { return d.dead || d.live; }
+__device__ __forceinline__ bool batch_gone(const plx_forward_desc& d, int, int p) { return d.dead && d.dead[p]; }
+__device__ __forceinline__ bool batch_gone(const plx_bwd_batch_desc& d, int e, int p) {
+  return (d.dead && d.dead[p]) || (d.live && !d.live[e]);
+}
 __host__ __device__ __forceinline__ const float* batch_rows(const plx_forward_desc& d) { return d.x; }
 __host__ __device__ __forceinline__ const float* batch_rows(const plx_bwd_batch_desc& d) { return d.g; }
 
@@ -877,7 +882,6 @@ __device__ __forceinline__ void batch_row(const D& d, int B) {
   const int b = (static_cast<int>(blockIdx.y) * 64 + lane) * V;
   const float* x = batch_rows(d) + (b < B ? b : B - V);  // every lane's loads stay in its row
   const int32_t* other = batch_other(d);
-  const uint8_t* dead = batch_dead(d);
   BatchLane<V> s;
 #pragma unroll
   for (int j = 0; j < V; ++j) s.v[j] = ident;
@@ -885,9 +889,9 @@ __device__ __forceinline__ void batch_row(const D& d, int B) {
     float w = 0.0f;  // entry c + lane of the chunk at c (past the row's end: its last one)
     int gone = 0;
     auto load_chunk = [&](int c) {
-      const int p = batch_pos(d, min(c + lane, e1 - 1));
+      const int e = min(c + lane, e1 - 1), p = batch_pos(d, e);
       w = d.weight[p];
-      if (!PLAIN) gone = dead ? dead[p] : 0;
+      if (!PLAIN) gone = batch_gone(d, e, p);
     };
     int ia[U], ib[U];
     BatchLane<V> ra[U], rb[U];
@@ -942,7 +946,7 @@ __device__ __forceinline__ void batch_row(const D& d, int B) {
 
 template <int M, class D, int V>
 __global__ __launch_bounds__(64) void k_batch_rows(D d, int32_t B) {
-  if (d.map.flags == 0 && !batch_dead(d))
+  if (d.map.flags == 0 && !batch_skips(d))
     batch_row<M, D, V, true>(d, B);
   else
     batch_row<M, D, V, false>(d, B);
@@ -969,7 +973,6 @@ __global__ __launch_bounds__(kBatchBlock) void k_batch_groups(D d, int32_t B) {
   const int smp = static_cast<int>(threadIdx.x) % kGroup, sub = static_cast<int>(threadIdx.x) / kGroup;
   const int b = b0 + smp, bl = b < B ? b : B - 1;  // every lane's loads stay in its row
   const float* x = batch_rows(d);
-  const uint8_t* dead = batch_dead(d);
   constexpr int kStep = kBatchBlock / kGroup;
   float wv[kGroupPer], xv[kGroupPer];
   bool use[kGroupPer];
@@ -982,7 +985,7 @@ __global__ __launch_bounds__(kBatchBlock) void k_batch_groups(D d, int32_t B) {
       o[i] = batch_other(d)[at];
       const int p = batch_pos(d, at);
       wv[i] = d.weight[p];
-      use[i] = e < e1 && !(dead && dead[p]);
+      use[i] = e < e1 && !batch_gone(d, at, p);
     }
 #pragma unroll
     for (int i = 0; i < kGroupPer; ++i) xv[i] = x[static_cast<int64_t>(o[i]) * B + bl];
@@ -2129,6 +2132,8 @@ int plx_backward_batch(const plx_bwd_batch_desc* d, void* stream) {
 int plx_backward_lists(const plx_bwd_batch_desc* d, void* stream) {
   if (!d) return fail(PLX_ERR_INVALID, "plx_backward_lists: null descriptor");
   if (d->batch != 1) return fail(PLX_ERR_INVALID, "plx_backward_lists: batch must be 1");
+  if (d->pos || d->dead)
+    return fail(PLX_ERR_INVALID, "plx_backward_lists: pos and dead must be null (weight and live are in list order)");
   if (d->nrows < 0) return fail(PLX_ERR_INVALID, "plx_backward_lists: negative nrows");
   if (d->nrows == 0) return PLX_OK;
   if (!d->row_unit || !d->row_ptr || !d->dst || !d->weight || !d->g)

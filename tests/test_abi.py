@@ -87,6 +87,14 @@ def test_argument_errors_are_reported_not_raised(lib) -> None:
     bd = _lib.plx_bwd_batch_desc()
     bd.batch, bd.nrows = 2, 0
     assert lib.plx_backward_batch(bd, None) == 0
+    bd.batch = 1
+    assert lib.plx_backward_lists(bd, None) == 0
+    for field in ("pos", "dead"):  # fields that only the batched backward reads
+        ld = _lib.plx_bwd_batch_desc()
+        ld.batch = 1
+        setattr(ld, field, 16)
+        assert lib.plx_backward_lists(ld, None) == 1
+        assert b"pos and dead must be null" in lib.plx_last_error()
     ud = _lib.plx_update_desc()
     ud.n = 5
     assert lib.plx_update_batch(ud, 2, None) == 1
