@@ -1404,12 +1404,13 @@ __global__ __launch_bounds__(kBatchBlock) void k_spread_cols(int64_t n, int32_t 
     *out = w;
 }
 
-// The batch's inputs into their units' rows: dst[ids[k] * B + b] = x[b * n + k].
-__global__ __launch_bounds__(kBatchBlock) void k_scatter_batch(int32_t n, int32_t B, const int32_t* ids, const float* x,
-                                                               float* dst) {
+// The batch's inputs into their units' rows: dst[ids[k] * B + b] = x[b * n + k],
+// for the inputs k in [k0, k1).
+__global__ __launch_bounds__(kBatchBlock) void k_scatter_batch(int32_t n, int32_t k0, int32_t k1, int32_t B,
+                                                               const int32_t* ids, const float* x, float* dst) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * kBatchBlock + threadIdx.x;
-  if (i >= static_cast<int64_t>(n) * B) return;
-  const int k = static_cast<int>(i / B), b = static_cast<int>(i % B);
+  if (i >= static_cast<int64_t>(k1 - k0) * B) return;
+  const int k = k0 + static_cast<int>(i / B), b = static_cast<int>(i % B);
   dst[static_cast<int64_t>(ids[k]) * B + b] = x[static_cast<int64_t>(b) * n + k];
 }
 
@@ -1688,6 +1689,14 @@ __global__ void k_math(int32_t op, int64_t n, const float* x, const float* y, fl
 inline unsigned grid_for(int64_t n, int block) {
   return static_cast<unsigned>((n + block - 1) / block);
 }
+
+// Lanes of one launch of a kernel with a lane per value. A grid of 2^32 lanes
+// or more returns no error and leaves values unwritten (seen at 4.3G), so
+// entry points whose columns may hold that many cut them into launches of fewer.
+constexpr int64_t kLaunchLanes = int64_t{1} << 30;
+
+// Units of a launch that takes `lanes` lanes for each.
+inline int64_t units_per_launch(int64_t lanes) { return lanes < kLaunchLanes ? kLaunchLanes / lanes : 1; }
 
 // A program's sizes are in range; fields read at a fixed unit only where
 // the kernel honours them (the loss) and only among the program's fields.
@@ -2299,8 +2308,13 @@ int plx_reduce_cols(int64_t n, int32_t batch, int32_t ncols, const int32_t* mode
     c.dst[j] = static_cast<float*>(dst[j]);
     c.mode[j] = modes[j];
   }
-  const dim3 grid(grid_for(n, kReduceUnits), static_cast<unsigned>(ncols));
-  k_reduce_cols<<<grid, kBatchBlock, 0, static_cast<hipStream_t>(stream)>>>(n, batch, c);
+  const int64_t step = units_per_launch(kBatchBlock / kReduceUnits);
+  for (int64_t u = 0; u < n; u += step) {
+    const int64_t m = n - u < step ? n - u : step;
+    const dim3 grid(grid_for(m, kReduceUnits), static_cast<unsigned>(ncols));
+    k_reduce_cols<<<grid, kBatchBlock, 0, static_cast<hipStream_t>(stream)>>>(m, batch, c);
+    for (int32_t j = 0; j < ncols; ++j) c.src[j] += m * batch, c.dst[j] += m;
+  }
   return check_launch("plx_reduce_cols");
 }
 
@@ -2319,11 +2333,17 @@ int plx_spread_cols(int64_t n, int32_t batch, int32_t ncols, const void* const* 
     quads = quads && aligned16(dst[j]);
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid(grid_for(n * batch / (quads ? 4 : 1), kBatchBlock), static_cast<unsigned>(ncols));
-  if (quads)
-    k_spread_cols<4><<<grid, kBatchBlock, 0, s>>>(n, batch, c);
-  else
-    k_spread_cols<1><<<grid, kBatchBlock, 0, s>>>(n, batch, c);
+  const int64_t per = quads ? batch / 4 : batch;  // lanes of a unit
+  const int64_t step = units_per_launch(per);
+  for (int64_t u = 0; u < n; u += step) {
+    const int64_t m = n - u < step ? n - u : step;
+    const dim3 grid(grid_for(m * per, kBatchBlock), static_cast<unsigned>(ncols));
+    if (quads)
+      k_spread_cols<4><<<grid, kBatchBlock, 0, s>>>(m, batch, c);
+    else
+      k_spread_cols<1><<<grid, kBatchBlock, 0, s>>>(m, batch, c);
+    for (int32_t j = 0; j < ncols; ++j) c.src[j] += m, c.dst[j] += m * batch;
+  }
   return check_launch("plx_spread_cols");
 }
 
@@ -2331,8 +2351,12 @@ int plx_scatter_batch(int32_t n, int32_t batch, const int32_t* ids, const float*
   if (n < 0 || batch < 1) return fail(PLX_ERR_INVALID, "plx_scatter_batch: bad size");
   if (n == 0) return PLX_OK;
   if (!ids || !values || !dst) return fail(PLX_ERR_INVALID, "plx_scatter_batch: null pointer");
-  k_scatter_batch<<<grid_for(static_cast<int64_t>(n) * batch, kBatchBlock), kBatchBlock, 0,
-                    static_cast<hipStream_t>(stream)>>>(n, batch, ids, values, dst);
+  const int64_t step = units_per_launch(batch);
+  for (int64_t k = 0; k < n; k += step) {
+    const int32_t k1 = static_cast<int32_t>(n - k < step ? n : k + step);
+    k_scatter_batch<<<grid_for((k1 - k) * batch, kBatchBlock), kBatchBlock, 0, static_cast<hipStream_t>(stream)>>>(
+        n, static_cast<int32_t>(k), k1, batch, ids, values, dst);
+  }
   return check_launch("plx_scatter_batch");
 }
 

@@ -67,3 +67,40 @@ def test_columns_spread_scatter_and_reduce(n: int, batch: int, offset: int) -> N
             if mode == 0:
                 s /= np.float32(batch)
             assert _equal(got.cpu().numpy(), s), f"reduce mode {mode}"
+
+
+def test_columns_of_more_lanes_than_a_launch() -> None:
+    """A column of more than 2^32 values (one lane each: an odd batch), and
+    more units than one reduction launch takes."""
+    free, _ = torch.cuda.mem_get_info(DEV)
+    if free < 60 << 30:
+        pytest.skip("needs two 17 GB columns")
+    n, batch, part = 1_048_577, 4099, 8192
+    col = (torch.arange(n, device=DEV) % 8191).float()
+    out = torch.zeros((n, batch), device=DEV)
+    src_p, out_p = _pointers([col]), _pointers([out])
+    print(f"columns {n} batch {batch}", flush=True)
+    _lib.call("plx_spread_cols", n, batch, 1, ctypes.addressof(src_p), ctypes.addressof(out_p), None)
+    for u in range(0, n, part):
+        assert bool((out[u : u + part] == col[u : u + part, None]).all()), f"spread, units {u} .."
+    ids = torch.randperm(n, device=DEV).to(torch.int32)
+    x = torch.empty((batch, n), device=DEV)
+    k = torch.arange(n, device=DEV)
+    for b in range(0, batch, 64):
+        bs = torch.arange(b, min(b + 64, batch), device=DEV)
+        x[b : b + 64] = ((k[None] * 31 + bs[:, None] * 7) % 65521).float()
+    _lib.call("plx_scatter_batch", n, batch, ids.data_ptr(), x.data_ptr(), out.data_ptr(), None)
+    for u in range(0, n, part):
+        assert torch.equal(out[ids[u : u + part].long()], x[:, u : u + part].t()), f"scatter, inputs {u} .."
+    del out, x
+    n = (1 << 28) + 17
+    cols = (torch.arange(2 * n, device=DEV) % 4093).float()
+    red = [torch.zeros(n, device=DEV) for _ in range(3)]
+    modes = (ctypes.c_int32 * 3)(0, 1, 2)  # MEAN, SUM, FIRST
+    src_p, red_p = _pointers([cols] * 3), _pointers(red)
+    print(f"reduction of {n} units", flush=True)
+    _lib.call("plx_reduce_cols", n, 2, 3, ctypes.addressof(modes), ctypes.addressof(src_p), ctypes.addressof(red_p),
+              None)
+    both = cols[::2] + cols[1::2]
+    for got, want in zip(red, (both / 2, both, cols[::2])):
+        assert torch.equal(got, want)
