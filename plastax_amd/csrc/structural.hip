@@ -1942,9 +1942,17 @@ int plx_gen_fold(const plx_gen_fold_desc* d, void* stream) {
       return fail(PLX_ERR_INVALID, "plx_gen_fold: bad accumulator column or monoid");
   if (d->batch == 1) {
     const int rows = gen_fold_rows(d->nrows, plx_detail::cu_count());
-    const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(d->nrows) + rows - 1) / rows);
     const size_t lds = kGenWin * (sizeof(float) * static_cast<size_t>(d->ncomp) + 1);
-    hipLaunchKernelGGL(k_gen_fold, dim3(grid), dim3(kBlock), lds, static_cast<hipStream_t>(stream), *d, rows);
+    // (at most 2^22 workgroups a launch: 2^30 lanes. A grid of 2^32, 2^30 rows
+    // at 64 a workgroup, returns no error and leaves rows out.)
+    plx_gen_fold_desc part = *d;
+    const int64_t step = static_cast<int64_t>(rows) << 22;
+    for (int64_t r = 0; r < d->nrows; r += step) {
+      part.nrows = static_cast<int32_t>(d->nrows - r < step ? d->nrows - r : step);
+      const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(part.nrows) + rows - 1) / rows);
+      hipLaunchKernelGGL(k_gen_fold, dim3(grid), dim3(kBlock), lds, static_cast<hipStream_t>(stream), part, rows);
+      part.row_unit += step, part.row_ptr += step;
+    }
     return check_launch("plx_gen_fold");
   }
   hipLaunchKernelGGL(k_gen_fold_batch, dim3(grid_for(d->nrows * d->batch)), dim3(kBlock), 0,

@@ -12,6 +12,7 @@ import torch
 import nets
 import plastax_amd as px
 import plastax_amd.numpy as jnp
+from plastax_amd import _lib
 from test_gpu_parity import assert_same_state
 
 pytestmark = pytest.mark.gpu
@@ -79,3 +80,24 @@ def test_generic_fold_blocks_match_the_oracle(oracle, width: int, fwd, prune: bo
         o.step(x)
         torch.cuda.synchronize()
         assert_same_state(static, state, o, f"step {k}")
+
+
+def test_generic_fold_of_more_rows_than_a_launch() -> None:
+    """2^30 rows and some, at 64 a workgroup of 256 lanes: every row's
+    accumulator takes its fold (no entries: the identity, 2 here)."""
+    dev = torch.device("cuda", 0)
+    n = (1 << 30) + 130
+    if torch.cuda.mem_get_info(dev)[0] < 40 << 30:
+        pytest.skip("needs three 4 GB columns")
+    print(f"generic fold of {n} rows", flush=True)
+    units = torch.arange(n, dtype=torch.int32, device=dev)
+    ptr = torch.zeros(n + 1, dtype=torch.int32, device=dev)
+    acc = (units % 1021).float()
+    ids = torch.zeros(4, dtype=torch.int32, device=dev)
+    d = _lib.plx_gen_fold_desc()
+    d.nrows, d.ncomp, d.num_units, d.batch, d.prog.nout = n, 1, n, 1, 1
+    d.monoid[0], d.identity[0], d.acc[0] = 1, 2.0, acc.data_ptr()  # product
+    d.row_unit, d.row_ptr, d.from_id = units.data_ptr(), ptr.data_ptr(), ids.data_ptr()
+    _lib.call("plx_gen_fold", d, None)
+    want = (units % 1021).float() * 2.0
+    assert torch.equal(acc, want)
