@@ -570,9 +570,17 @@ class Arena:
         shared = self.t_name if self.t_name in names and self.t_now and self.t_now[b] is not None else None
         if shared is not None and DEAD.name not in names:
             names.remove(shared)
-        for c in [c for c in names if self.cols[c].element_size() not in (1, 4)]:
+
+        def dense(c: str) -> bool:
+            """Whether a kernel can write column c through its pointer."""
+            return (bucket[c].is_contiguous() and bucket[c].dtype == self.cols[c].dtype
+                    and bucket[c].element_size() in (1, 4))
+
+        for c in [c for c in names if not dense(c)]:  # (a strided view of the caller's: written by torch)
             names.remove(c)
-            bucket[c][self.slot[base : base + n].long()] = self.cols[c][base : base + n]
+            at = self.slot[base : base + n]
+            own = (at >= 0).nonzero().squeeze(1)
+            bucket[c][at[own].long()] = self.cols[c][base : base + n][own]
         for c0 in range(0, len(names), _lib.PLX_MAX_SLOT_COLS):
             part = names[c0 : c0 + _lib.PLX_MAX_SLOT_COLS]
             cols = [self.cols[c] for c in part]
@@ -584,7 +592,9 @@ class Arena:
                 ctypes.addressof(src), ctypes.addressof(dst), ctypes.addressof(size),
                 sum(1 << j for j, c in enumerate(part) if c in (DEAD.name, shared)),
                 self.cols[DEAD.name].data_ptr() + base, self.lives[b], stream), "plx_write_slots")
-        if shared is not None:
+        if shared is not None and not (dense(shared) and dense(DEAD.name)):
+            bucket[shared][bucket[DEAD.name] == 0] = float(self.t_now[b])
+        elif shared is not None:
             _lib.check(lib.plx_fill_live(cap, bucket[DEAD.name].data_ptr(), float(self.t_now[b]),
                                          bucket[shared].data_ptr(), stream), "plx_fill_live")
 

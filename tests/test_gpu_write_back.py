@@ -102,3 +102,43 @@ def test_logical_view_after_kills_matches_the_oracle(oracle, mode: str, every: i
         if k % every == every - 1:
             print(f"write back {mode} step {k}", flush=True)
             assert_same_state(static, state, o, f"step {k}")
+
+
+@pytest.mark.parametrize("strided", [("weight",), ("dead", "opt/t"), ("dead", "weight", "opt/m", "opt/v", "opt/t")])
+def test_logical_columns_that_are_strided_views(oracle, strided: tuple[str, ...]) -> None:
+    """A caller's bucket columns that are strided views (the host-built layout
+    reads any): the copy back follows their strides and leaves the storage
+    between their elements alone."""
+    base = nets.make_trained_net("WS", nets.TanhForward(), nets.TanhBackward(), px.optim.adam(1e-2, nets.GRAD_PRE_ACT),
+                                 px.Propagation.TOPOLOGICAL)
+
+    class Net(base):
+        prune_conn = _Prune()
+
+    e = synth.c2_topological(seed=4, scale=512, layers=3)
+    g = {"step": np.int32(0)}
+    static, state = px.NetworkBuilder.from_edges(Net, e.num_units, e.src, e.dst, weights=e.weight,
+                                                 input_ids=e.input_ids, output_ids=e.output_ids, globals_=g,
+                                                 capacity_headroom=0.3, device="cuda")
+    o = nets.oracle_for(oracle, Net, static, state)
+    buckets, between = [], []
+    for bucket in state.conns:
+        new = dict(bucket)
+        for name in strided:
+            room = torch.full((2 * bucket[name].numel(),), 77, dtype=bucket[name].dtype, device=DEV)
+            new[name] = room[::2].copy_(bucket[name])
+            between.append(room[1::2])
+        buckets.append(new)
+    state.conns = tuple(buckets)
+    step = px.make_step(Net, static)
+    step.layout_build = "host"
+    rng = np.random.default_rng(5)
+    for k in range(3):
+        state.globals_ = o.globals_ = {"step": np.int32(k)}
+        x = rng.standard_normal(e.input_ids.size).astype(np.float32)
+        t = rng.standard_normal(e.output_ids.size).astype(np.float32)
+        print(f"write back, strided {strided}, step {k}", flush=True)
+        state = step(state, px.StepInputs(x, t)).state
+        o.step(x, t)
+        assert_same_state(static, state, o, f"step {k}")
+        assert all(bool((gap == 77).all()) for gap in between)
