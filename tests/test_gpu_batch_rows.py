@@ -1,8 +1,9 @@
-"""The batched forward and backward at the edges of their dispatch: levels of
-255 and 256 rows (sample groups, a wave per row), batches around a wave's
-samples (one and four per lane), rows of no, 16, 64, 65 and several hundred
-entries, with and without tombstones inside them -- bit for bit with the
-batched oracle."""
+"""The batched step at the edges of its levels' dispatch: 255 and 256 rows
+(sample groups, a wave per row), batches around a wave's samples (one and four
+per lane), forward rows of 1 to 399 entries (16, 64, 65 and 128 among them),
+backward rows of at most 9 and the outputs' empty ones, with and without
+tombstones inside them -- bit for bit with the batched oracle. (Empty forward
+rows, long backward rows and the other monoids: test_gpu_batch_entries.)"""
 
 from __future__ import annotations
 
