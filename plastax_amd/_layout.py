@@ -570,33 +570,36 @@ class Arena:
         shared = self.t_name if self.t_name in names and self.t_now and self.t_now[b] is not None else None
         if shared is not None and DEAD.name not in names:
             names.remove(shared)
-
-        def dense(c: str) -> bool:
-            """Whether a kernel can write column c through its pointer."""
-            return (bucket[c].is_contiguous() and bucket[c].dtype == self.cols[c].dtype
-                    and bucket[c].element_size() in (1, 4))
-
-        for c in [c for c in names if not dense(c)]:  # (a strided view of the caller's: written by torch)
-            names.remove(c)
+        # A kernel writes through the columns' pointers; a bucket's column that
+        # is a strided view of the caller's, or no 1- or 4-byte one, is written
+        # by torch.
+        todo = []
+        for c in names:
+            src, dst = self.cols[c], bucket[c]
+            size = src.element_size()
+            if (size == 1 or size == 4) and dst.dtype == src.dtype and dst.is_contiguous():
+                todo.append((c, src.data_ptr() + base * size, dst.data_ptr(), size))
+                continue
             at = self.slot[base : base + n]
             own = (at >= 0).nonzero().squeeze(1)
-            bucket[c][at[own].long()] = self.cols[c][base : base + n][own]
-        for c0 in range(0, len(names), _lib.PLX_MAX_SLOT_COLS):
-            part = names[c0 : c0 + _lib.PLX_MAX_SLOT_COLS]
-            cols = [self.cols[c] for c in part]
-            src = (ctypes.c_void_p * len(part))(*[c.data_ptr() + base * c.element_size() for c in cols])
-            dst = (ctypes.c_void_p * len(part))(*[bucket[c].data_ptr() for c in part])
-            size = (ctypes.c_int32 * len(part))(*[c.element_size() for c in cols])
+            dst[at[own].long()] = src[base : base + n][own]
+        for c0 in range(0, len(todo), _lib.PLX_MAX_SLOT_COLS):
+            part = todo[c0 : c0 + _lib.PLX_MAX_SLOT_COLS]
+            src = (ctypes.c_void_p * len(part))(*[p for _, p, _, _ in part])
+            dst = (ctypes.c_void_p * len(part))(*[p for _, _, p, _ in part])
+            size = (ctypes.c_int32 * len(part))(*[k for _, _, _, k in part])
             _lib.check(lib.plx_write_slots(
                 n, None if n_dev is None else n_dev.data_ptr(), self.slot.data_ptr() + 4 * base, cap, len(part),
                 ctypes.addressof(src), ctypes.addressof(dst), ctypes.addressof(size),
-                sum(1 << j for j, c in enumerate(part) if c in (DEAD.name, shared)),
+                sum(1 << j for j, col in enumerate(part) if col[0] in (DEAD.name, shared)),
                 self.cols[DEAD.name].data_ptr() + base, self.lives[b], stream), "plx_write_slots")
-        if shared is not None and not (dense(shared) and dense(DEAD.name)):
-            bucket[shared][bucket[DEAD.name] == 0] = float(self.t_now[b])
-        elif shared is not None:
-            _lib.check(lib.plx_fill_live(cap, bucket[DEAD.name].data_ptr(), float(self.t_now[b]),
-                                         bucket[shared].data_ptr(), stream), "plx_fill_live")
+        if shared is not None:
+            dead, col = bucket[DEAD.name], bucket[shared]
+            if dead.is_contiguous() and col.is_contiguous():
+                _lib.check(lib.plx_fill_live(cap, dead.data_ptr(), float(self.t_now[b]), col.data_ptr(), stream),
+                           "plx_fill_live")
+            else:
+                col[dead == 0] = float(self.t_now[b])
 
     def _write_logical_host(self, conns: tuple[Columns, ...]) -> None:
         """write_logical of an arena laid out on the CPU: every column (unit
