@@ -630,8 +630,8 @@ PLX_EXPORT int plx_forward_bucket_compiled(void* handle, const plx_forward_desc*
 
 /* One bucket of a generic pass (a map outside the product form, one float32
  * component or a tuple with a tuple of monoids: sweep.py:113-180 / :343-399
- * with any `map` and `combine`): for every row r (one thread each), unit u =
- * row_unit[r], its entries j in [row_ptr[r], row_ptr[r+1]) in order, each at
+ * with any `map` and `combine`): for every row r, unit u = row_unit[r], its
+ * entries j in [row_ptr[r], row_ptr[r+1]) in order, each at
  * physical position p = entry_pos ? entry_pos[j] : j, skipped where dead[p]
  * (dead optional): the map program (`prog`, ncomp float32 outputs) runs as
  * the PLX_SITES_EDGE site s = p - base (its connection columns start at

@@ -9,7 +9,7 @@ Flags that carry meaning:
   sum of the step rounds to float32 on its own, exactly as the reference's
   jnp operations do, so the device trajectory can be compared bit for bit.
 - ``-Xclang -target-feature -Xclang -packed-fp32-ops``: no packed float32
-  instructions (their results have been unreliable on this pool).
+  instructions (some of their forms have given wrong results on this GPU).
 """
 
 from __future__ import annotations

@@ -800,11 +800,12 @@ __device__ __forceinline__ float fold_in_order(const float* v, int len, float s)
 }
 
 // ---------------------------------------------------------------------------
-// Batched steps. Unit columns are [num_units][B]: a row of the forward or
-// the backward is one workgroup whose lanes are the samples, so the gathered
-// unit row (x[src * B ..] or g[dst * B ..]) is one coalesced B-wide read,
-// while FROM_ID / TO_ID / WEIGHT / DEAD are uniform across the workgroup.
-// Each lane folds its sample's terms in the streaming step's order.
+// Batched steps. Unit columns are [num_units][B]: the gathered unit row
+// (x[src * B ..] or g[dst * B ..]) is a coalesced B-wide read whose lanes are
+// the samples. A row of the forward or the backward is a wave per 64 or 256
+// samples (k_batch_rows), in levels of few rows a workgroup per 16
+// (k_batch_groups). Each sample's terms are folded in the streaming step's
+// order.
 // ---------------------------------------------------------------------------
 constexpr int kBatchBlock = 256;
 constexpr int kBatchUnroll = 8;  // unit rows loaded together by a wave of k_batch_rows
@@ -952,9 +953,11 @@ __global__ __launch_bounds__(64) void k_batch_rows(D d, int32_t B) {
     batch_row<M, D, V, false>(d, B);
 }
 
-// Levels of few rows: a workgroup per (row, kGroup samples), whose lanes form the terms of kGroupWin
-// entries side by side (a lane per sample and entry) into LDS, where a lane
-// per sample folds them in order while the next window's loads are in flight.
+// Levels of few rows: a workgroup per (row, kGroup samples), whose lanes form
+// the terms of kGroupWin entries side by side (a lane per sample and entry)
+// into LDS, where a lane per sample folds them in order while the next
+// window's loads are in flight. A skipped entry's term is the identity, which
+// leaves every monoid's running value as it is.
 // With a 256-lane workgroup per row such a level waited for one chain of id
 // and row loads per sixteen entries (ten rows of 410 edges, 256 samples:
 // 37.6 us, ten CUs busy; 11.0 in groups).
@@ -1070,7 +1073,9 @@ __global__ void k_gather_edges(int64_t n, const int32_t* pos, const float* weigh
   if (out_live) out_live[j] = dead ? (dead[p] == 0) : 1;
 }
 
-// The batched update, one lane per position: its batch-mean gradient is
+// The batched update, one lane per position (plx_update_batch, for a caller
+// without tiles: a batched step builds them and runs plx_update_batch_tiles
+// alone): its batch-mean gradient is
 // stat_0 + stat_1 + ... in sample order, / B (phases.py:462-471), with
 // stat_b = gfield[dst * B + b] * act[src * B + b], then the update rule.
 // The two B-wide rows are read in 16-byte slices, 32 samples' slices in

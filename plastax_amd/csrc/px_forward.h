@@ -375,9 +375,10 @@ constexpr int kFwdPerCU = PLX_FWD_PER_CU;  // workgroups per CU in the persisten
 // before, this rule after: 4,096 rows of 410 edges 83 -> 10.5 us; 2,048 rows
 // of 73 17.1 -> 7.0; 30,011 of 37 14.0 -> 9.6; 32,768 of 73 20.6 -> 13.2;
 // 131,072 of 73 (still 256 rows) 26.7 -> 26.2 by the fold's longer reads.
-// Twice as many blocks (two waves of workgroups) were slower everywhere
-// (10.9 / 13.3 / 15.0 us for the last three but one), and so were tables cut
-// to a share of the block's edges (7.5 against 7.2).
+// Twice as many blocks (two waves of workgroups) gain nothing at any of them
+// (launches one after another over random rows, this rule -> twice as many:
+// 2,048 rows of 73 edges 5.8 -> 6.0 us, 4,096 of 410 8.4 -> 8.4, 30,011 of 37
+// 7.0 -> 9.2, 32,768 of 73 10.6 -> 11.1).
 inline int fwd_block_rows(int nrows, int ncu) {
   const int two = (nrows + kFwdPerCU * ncu - 1) / (kFwdPerCU * ncu);
   const int one = (nrows + ncu - 1) / ncu;

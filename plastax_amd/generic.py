@@ -9,7 +9,8 @@ reference's examples xmc.py, upgd.py, cbp.py) -- runs here:
 
 - the map is traced into an edge program with one float32 output per
   accumulator component (``_site.trace_pass_map``);
-- ``plx_gen_fold`` folds each row's entries in order, one thread per row:
+- ``plx_gen_fold`` evaluates the map of a block of rows' entries side by
+  side and folds each row's values in order, a lane per row and component:
   a forward row is a destination, its entries the slab range of its
   in-edges (slot order); a backward row a source, its entries its out-edges
   in slot order (the churn layout's lists, or on a tiled arena the
@@ -27,8 +28,8 @@ level from the identity, then level b after bucket b down to 1 (PIPELINE:
 every unit after one sweep).
 
 Under a batched step (``batch`` B > 1) every unit column the programs read
-and the accumulators are ``[num_units][B]``: the fold runs one thread per
-(row, sample), the apply one site per (finalized unit, sample), and each
+and the accumulators are ``[num_units][B]``: the fold runs one lane per
+(row, sample), evaluating and folding its entries one after another, the apply one site per (finalized unit, sample), and each
 sample's writes land at ``unit * B + sample`` (step.py:443-447 runs the
 pass per sample against the shared connections).
 """

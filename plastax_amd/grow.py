@@ -368,7 +368,8 @@ def unflatten(flat: Columns, offs: list[int]) -> tuple[Columns, ...]:
 
 class PruneConnPhase:
     """``dead |= predicate(u, c, cid, g)`` over every slot of every bucket
-    (phases.py:1444-1498), one site-program launch per bucket."""
+    (phases.py:1444-1498): one site-program launch per bucket on the logical
+    arena, one over the slab on the physical one (see run_physical)."""
 
     def __init__(self, net: Any, static: Any, globals_: Any) -> None:
         self.static = static
@@ -404,11 +405,11 @@ class PruneConnPhase:
         reads_ids = bool({FROM_ID.name, TO_ID.name} & set(self.prog.conn_fields))
         logical = arena.logical_ids() if reads_ids and not churn else None
         # The buckets lie one after another in one slab, so one launch takes
-        # them all (what it reads past a bucket's end is dead): 16.8M edges
-        # in seven buckets take 22.3 us, 40.9 in seven launches, whose host
-        # time was 34 us each. Only what a
-        # kill stamps can differ between buckets (one without live edges
-        # stamps nothing).
+        # them all (what it reads past a bucket's end is dead): 16.8M edges in
+        # seven buckets take 22.3 us, and 40.9 in seven launches, each of which
+        # also cost the host 34 us. Only what a kill stamps can differ between
+        # buckets (one without live edges stamps nothing); where it does, each
+        # bucket takes a launch of its own.
         spans = []
         stamps = [arena.stamp_target(b) for b in range(arena.num_buckets)]
         if len({(t is None, v) for (t, v), live in zip(stamps, arena.lives) if live}) > 1:
