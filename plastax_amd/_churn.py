@@ -398,13 +398,14 @@ class ChurnArena(Arena):
         (the slots dead at layout time were never written by the step): the
         columns a step wrote since the last such copy (a prune: DEAD and the
         step count it stamps), or all of them."""
-        written, self._written = self._written, set()
+        written = self._written
         if written is not None and written <= {DEAD.name, self.t_name}:
             self._write_kills(conns, written)
-            return
-        for b, bucket in enumerate(conns):
-            # positions [0, live count) to their logical slots (the count on the device)
-            self._write_bucket(b, bucket, written, self.lives[b], n_dev=self.live_dev[b])
+        else:
+            for b, bucket in enumerate(conns):
+                # positions [0, live count) to their logical slots (the count on the device)
+                self._write_bucket(b, bucket, written, self.lives[b], n_dev=self.live_dev[b])
+        self._written = set()  # (a copy that failed is due again at the next read)
 
 
 def _side(side, n: int, limit: int, ids: torch.Tensor, key1: torch.Tensor, key2: torch.Tensor | None,

@@ -542,14 +542,15 @@ class Arena:
         """The columns a step wrote since the last such copy, scattered back
         into the logical buckets (the logical view's other columns are in
         step: a layout's edges, ids and slots never change in place)."""
-        written, self._written = self._written, set()
+        written = self._written
         if self.device.type != "cuda":
             self._write_logical_host(conns)
-            return
-        for b, bucket in enumerate(conns):
-            # What a step writes lies among the positions live at layout time;
-            # a caller that names no columns may have written any.
-            self._write_bucket(b, bucket, written, self.caps[b] if written is None else self.lives[b])
+        else:
+            for b, bucket in enumerate(conns):
+                # What a step writes lies among the positions live at layout
+                # time; a caller that names no columns may have written any.
+                self._write_bucket(b, bucket, written, self.caps[b] if written is None else self.lives[b])
+        self._written = set()  # (a copy that failed is due again at the next read)
 
     def _write_bucket(self, b: int, bucket: Columns, written: set | None, n: int,
                       n_dev: torch.Tensor | None = None) -> None:
