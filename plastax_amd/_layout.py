@@ -545,6 +545,9 @@ class Arena:
         written = self._written
         if self.device.type != "cuda":
             self._write_logical_host(conns)
+        elif self.device.index not in (None, torch.cuda.current_device()):
+            with torch.cuda.device(self.device):  # (the kernels launch on the current device)
+                self.write_logical(conns)
         else:
             for b, bucket in enumerate(conns):
                 # What a step writes lies among the positions live at layout

@@ -1,6 +1,7 @@
 """The copy back into the logical buckets, host side (no kernel runs: the
 library is a stand-in): a copy that fails is due again at the next read, on
-either layout."""
+either layout; a tiled arena's view read while another device is current is
+copied on the arena's."""
 
 from __future__ import annotations
 
@@ -32,6 +33,7 @@ class _StandIn:
 def _state(monkeypatch, cls) -> tuple[NetworkState, Arena, _StandIn]:
     lib = _StandIn()
     monkeypatch.setattr(_lib, "load", lambda: lib)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: types.SimpleNamespace(cuda_stream=0))
     dtypes = dict(from_id=torch.int32, to_id=torch.int32, weight=torch.float32, dead=torch.uint8)
     conns = tuple({k: torch.zeros(8, dtype=t) for k, t in dtypes.items()} for _ in range(3))
@@ -64,3 +66,26 @@ def test_a_failed_copy_back_is_due_again(monkeypatch, cls, columns) -> None:
     state.conns
     assert lib.writes == 3  # and then the view is in step
     assert arena._written == set()
+
+
+def test_the_copy_back_runs_on_the_arenas_device(monkeypatch) -> None:
+    state, arena, lib = _state(monkeypatch, Arena)
+    current = [1]
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[-1])
+
+    class On:
+        def __init__(self, device) -> None:
+            self.index = torch.device(device).index
+
+        def __enter__(self) -> None:
+            current.append(self.index)
+
+        def __exit__(self, *exc) -> None:
+            current.pop()
+
+    monkeypatch.setattr(torch.cuda, "device", On)
+    on = []
+    monkeypatch.setattr(lib, "plx_write_slots", lambda *args: on.append(current[-1]) or 0, raising=False)
+    state._mark_ahead({"weight"})
+    state.conns
+    assert on == [0, 0, 0] and current == [1] and arena._written == set()
